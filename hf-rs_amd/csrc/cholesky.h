@@ -18,7 +18,7 @@ struct CholeskyInfo {
 // Factors of the AO ERIs of shells orb (n functions) to residual diagonal
 // threshold, with at most budget bytes of packed factors (the reference's
 // rule: 8 np (K + 2) <= budget before row K is added), on stream st; the
-// result is d_B = [rank][n][n] (each factor unpacked, symmetric).
+// result is d_B, rank rows of the tiled layout (df_tiles.h).
 void cholesky_factors(const std::vector<Shell>& orb, int n, hipStream_t st, Blas& bl, double threshold, double budget,
                       DevBuf& d_B, int& rank, CholeskyInfo& info);
 

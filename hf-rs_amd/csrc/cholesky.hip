@@ -17,8 +17,8 @@
 // so far (L as an np x K column-major matrix, the pivot's entries read with
 // stride np); one workgroup updates the residual diagonal, checks it and
 // picks the next pivot, so each step returns one (pivot, maximum, flag)
-// triple to the host.  The factors end as the unpacked [rank][n][n] tensor
-// the density-fitting J/K kernels read (src/df.rs:121 keeps them packed).
+// triple to the host.  The factors end in the tiled layout that the
+// density-fitting J/K kernels read (src/df.rs:121 keeps them packed).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "cholesky.h"
+#include "df_tiles.h"
 #include "la_device.h"
 
 namespace hfg {
@@ -153,12 +154,16 @@ __global__ __launch_bounds__(1024) void k_chol_step(double* __restrict__ diag, s
   }
 }
 
-// B[K][p][q] = B[K][q][p] = L[K][cpair(p, q)].
-__global__ void k_chol_unpack(const double* __restrict__ L, int rank, int n, double* __restrict__ B) {
-  const size_t nn = (size_t)n * n, np = (size_t)n * (n + 1) / 2, total = (size_t)rank * nn;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-    const size_t K = i / nn, pq = i % nn;
-    B[i] = L[K * np + cpair(pq / n, pq % n)];
+// Packed rows L[K] -> the tiled factor (df_tiles.h).
+__global__ void k_chol_tiles(const double* __restrict__ L, int rank, int n, size_t npt, double* __restrict__ B) {
+  const size_t np = (size_t)n * (n + 1) / 2, tile = TL * TL;
+  const int K = blockIdx.y, t = blockIdx.x;  // one tile (I, J) of row K
+  int I = 0;
+  while ((I + 1) * (I + 2) / 2 <= t) ++I;
+  const int J = t - I * (I + 1) / 2;
+  for (int e = threadIdx.x; e < (int)tile; e += blockDim.x) {
+    const int i = I * TL + e / TL, j = J * TL + e % TL;
+    B[(size_t)K * npt + (size_t)t * tile + e] = (i < n && j < n) ? L[K * np + cpair(i, j)] : 0.0;
   }
 }
 
@@ -410,9 +415,11 @@ void cholesky_factors(const std::vector<Shell>& orb, int n, hipStream_t st, Blas
     throw HfgError{HFG_INTEGRAL, "pivoted Cholesky ERI decomposition: threshold exceeds every ERI diagonal; no "
                                  "Cholesky vectors were generated"};
   info.rank = rank;
-  const size_t nn = (size_t)n * n;
-  d_B.alloc((size_t)rank * nn * 8);
-  hipLaunchKernelGGL(k_chol_unpack, dim3(4096), dim3(256), 0, st, d_L.p, rank, n, d_B.as<double>());
+  const size_t npt = tiled_size(n);
+  d_B.alloc((size_t)rank * npt * 8);
+  for (int k0 = 0; k0 < rank; k0 += 65535)
+    hipLaunchKernelGGL(k_chol_tiles, dim3((unsigned)(npt / (TL * TL)), (unsigned)std::min(rank - k0, 65535)), dim3(256),
+                       0, st, d_L.p + k0 * np, rank, n, npt, d_B.as<double>() + k0 * npt);
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(st));
 }

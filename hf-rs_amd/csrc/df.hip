@@ -7,11 +7,10 @@
 // three_center_integrals, DfTensor::build, coulomb_exchange_rhf) and
 // run_factorized_rhf (src/hf_variants/ri_df_hf.rs:160-263).  The integrals are
 // the generated Head-Gordon-Pople blocks with the auxiliary shell paired with
-// the exponent-0 unit function (src/df.rs:30-40); B is kept unpacked,
-// [rank][n][n], so that DF-J is two FP64 GEMVs over B (HBM-bound) and DF-K is
-// one batched GEMM A_Q = B_Q C plus one GEMM K = 2 A' A'^T over the
-// rank*n_occ index (FP64 matrix cores through rocBLAS).
-#include <hip/hip_bf16.h>
+// the exponent-0 unit function (src/df.rs:30-40).  B is kept as the tiles of its
+// rows' lower triangles (df_tiles.h), formed one chunk of tile rows at a time;
+// DF-J is two passes over B (HBM-bound), DF-K the matrix-core products of
+// df_mfma.hip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,6 +28,7 @@
 
 #include "../../include/hfg.h"
 #include "cholesky.h"
+#include "df_tiles.h"
 #include "engine.h"
 #include "la_device.h"
 #include "rhf.h"
@@ -36,7 +36,7 @@
 
 namespace hfg {
 
-// Block element -> 3-index tensor T[P][mu][nu] (both mu nu orders), scaled.
+// Where a 3-index block's elements go.
 struct Scatter3 {
   long long off;
   int aux_bra;        // 1: block is (P 1|a b), else (a b|P 1)
@@ -44,41 +44,14 @@ struct Scatter3 {
   int mu0, nu0, p0;   // AO offsets of first / second orbital shell and aux shell
 };
 
+// Block element -> T[P][tiled_at(i, j) - c0] of a chunk of tile rows [I0, I1)
+// (cols doubles a row, c0 its first tile's position), i >= j; on the tiles of
+// the diagonal the transposed element as well.  A block of one shell with
+// itself writes only its a >= b elements, and elements of other tile rows
+// belong to another chunk, so every entry is written once.
 __global__ void k_scatter3(const Scatter3* __restrict__ d, int ntask, const double* __restrict__ blk,
                            const double* __restrict__ so, const double* __restrict__ sx, double* __restrict__ T,
-                           int n) {
-  const int t = blockIdx.x;
-  if (t >= ntask) return;
-  const Scatter3 s = d[t];
-  const int tot = s.na * s.nb * s.np;
-  const size_t nn = (size_t)n * n;
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int a, b, p;
-    if (s.aux_bra) {
-      p = e / (s.na * s.nb);
-      const int r = e - p * s.na * s.nb;
-      a = r / s.nb;
-      b = r - a * s.nb;
-    } else {
-      a = e / (s.nb * s.np);
-      const int r = e - a * s.nb * s.np;
-      b = r / s.np;
-      p = r - b * s.np;
-    }
-    const int mu = s.mu0 + a, nu = s.nu0 + b, P = s.p0 + p;
-    const double v = blk[s.off + e] * so[mu] * so[nu] * sx[P];
-    T[(size_t)P * nn + (size_t)mu * n + nu] = v;
-    T[(size_t)P * nn + (size_t)nu * n + mu] = v;
-  }
-}
-
-// Packed layout: column ij = i(i+1)/2 + j (i >= j) of the pair (mu, nu),
-// the src/scf.rs:221-235 compound index.  Block element -> T[P][ij - c0] of a
-// column chunk (cols wide); a block of one shell with itself writes only its
-// a >= b elements, so every entry is written once.
-__global__ void k_scatter3p(const Scatter3* __restrict__ d, int ntask, const double* __restrict__ blk,
-                            const double* __restrict__ so, const double* __restrict__ sx, double* __restrict__ T,
-                            long long c0, long long cols) {
+                           int I0, int I1, size_t c0, size_t cols) {
   const int t = blockIdx.x;
   if (t >= ntask) return;
   const Scatter3 s = d[t];
@@ -99,22 +72,33 @@ __global__ void k_scatter3p(const Scatter3* __restrict__ d, int ntask, const dou
     }
     if (diag && a < b) continue;
     const int mu = s.mu0 + a, nu = s.nu0 + b, P = s.p0 + p;
-    const long long i = mu > nu ? mu : nu, j = mu > nu ? nu : mu;
-    T[(size_t)P * cols + (size_t)(i * (i + 1) / 2 + j - c0)] = blk[s.off + e] * so[mu] * so[nu] * sx[P];
+    const int i = mu > nu ? mu : nu, j = mu > nu ? nu : mu;
+    if (i / TL < I0 || i / TL >= I1) continue;
+    const double v = blk[s.off + e] * so[mu] * so[nu] * sx[P];
+    double* row = T + (size_t)P * cols;
+    row[tiled_at(i, j) - c0] = v;
+    if (i / TL == j / TL) row[tiled_at(j, i) - c0] = v;
   }
 }
 
-// Symmetric n x n -> packed with the off-diagonal doubled: sum_ij X_ij Y_ij
-// = sum_(i>=j) packed(X)_ij Y_ij for symmetric X, Y.
-__global__ void k_pack_sym2(const double* __restrict__ X, int n, double* __restrict__ Xp) {
-  const size_t ij = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t np = (size_t)n * (n + 1) / 2;
-  if (ij >= np) return;
-  int ii = (int)((sqrt(8.0 * (double)ij + 1.0) - 1.0) * 0.5);
-  while ((size_t)ii * (ii + 1) / 2 > ij) --ii;
-  while ((size_t)(ii + 1) * (ii + 2) / 2 <= ij) ++ii;
-  const int j = (int)(ij - (size_t)ii * (ii + 1) / 2);
-  Xp[ij] = (ii == j ? 1.0 : 2.0) * X[(size_t)ii * n + j];
+// Position x of the tiled layout -> its (i, j); i or j past n: padding.
+__device__ __forceinline__ void tiled_ij(size_t x, int& i, int& j) {
+  const int t = (int)(x / (TL * TL)), r = (int)(x % (TL * TL));
+  int I = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (I * (I + 1) / 2 > t) --I;
+  while ((I + 1) * (I + 2) / 2 <= t) ++I;
+  i = I * TL + r / TL;
+  j = (t - I * (I + 1) / 2) * TL + r % TL;
+}
+
+// Symmetric n x n -> tiled, doubled off the diagonal tiles: sum_ij X_ij Y_ij =
+// sum_x tiled2(X)_x tiled(Y)_x for symmetric X, Y.
+__global__ void k_tile_sym2(const double* __restrict__ X, int n, size_t npt, double* __restrict__ Xt) {
+  const size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (x >= npt) return;
+  int i, j;
+  tiled_ij(x, i, j);
+  Xt[x] = (i < n && j < n) ? (i / TL == j / TL ? 1.0 : 2.0) * X[(size_t)i * n + j] : 0.0;
 }
 
 // d[Q] = sum_j B[Q][j] v[j] over the nc columns of rows Q (row stride ld), four
@@ -168,63 +152,12 @@ __global__ __launch_bounds__(RD_NT) void k_rowdot(const double* __restrict__ B, 
   if (t < RD_ROWS && q0 + t < rows) d[q0 + t] = red[t][0];
 }
 
-// Packed -> symmetric n x n.
-__global__ void k_unpack_sym(const double* __restrict__ Xp, int n, double* __restrict__ X) {
+// Tiled -> symmetric n x n.
+__global__ void k_untile_sym(const double* __restrict__ Xt, int n, double* __restrict__ X) {
   const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (size_t)n * n) return;
   const int i = (int)(idx / n), j = (int)(idx - (size_t)i * n);
-  const int a = i > j ? i : j, b = i > j ? j : i;
-  X[idx] = Xp[(size_t)a * (a + 1) / 2 + b];
-}
-
-// Rows q < nq of packed B (row stride np) -> nq symmetric n x n matrices of
-// type T (double, float, or the two BF16 parts of a split, hi and lo), by
-// 64 x 64 tiles through LDS, so that both the packed reads (along j of a row
-// i >= j) and the two writes (row i of the lower tile, row j of its
-// transpose) are coalesced.  grid (lower tiles, nq), 256 threads.
-template <class T>
-__global__ __launch_bounds__(256) void k_unpack_tiles(const double* __restrict__ Bp, int n, size_t np, int nt,
-                                                      T* __restrict__ out, __hip_bfloat16* __restrict__ lo) {
-  __shared__ double tile[64 * 65];
-  int ti = 0, rem = blockIdx.x;  // lower tile (ti >= tj), row-major over the triangle
-  while (rem > ti) {
-    rem -= ti + 1;
-    ++ti;
-  }
-  const int tj = rem;
-  const int q = blockIdx.y;
-  const double* B = Bp + (size_t)q * np;
-  const size_t nn = (size_t)n * n;
-  T* O = out + (size_t)q * nn;
-  __hip_bfloat16* Lo = lo ? lo + (size_t)q * nn : nullptr;
-  const int i0 = ti * 64, j0 = tj * 64, t = threadIdx.x;
-  const bool diag = ti == tj;
-  auto put = [&](size_t at, double v) {
-    if constexpr (std::is_same<T, __hip_bfloat16>::value) {  // as k_split_bf16
-      const float f = (float)v;
-      const __hip_bfloat16 h = __float2bfloat16(f);
-      O[at] = h;
-      Lo[at] = __float2bfloat16(f - __bfloat162float(h));
-    } else {
-      O[at] = (T)v;
-    }
-  };
-  for (int r = 0; r < 16; ++r) {
-    const int li = (t >> 6) + 4 * r, lj = t & 63;
-    const int i = i0 + li, j = j0 + lj;
-    double v = 0.0;
-    if (i < n && j < n && (!diag || j <= i)) {
-      v = B[(size_t)i * (i + 1) / 2 + j];
-      put((size_t)i * n + j, v);
-    }
-    tile[li * 65 + lj] = v;
-  }
-  __syncthreads();
-  for (int r = 0; r < 16; ++r) {
-    const int lj = (t >> 6) + 4 * r, li = t & 63;  // out row j, along i
-    const int i = i0 + li, j = j0 + lj;
-    if (i < n && j < n && (!diag || i > j)) put((size_t)j * n + i, tile[li * 65 + lj]);
-  }
+  X[idx] = Xt[i > j ? tiled_at(i, j) : tiled_at(j, i)];
 }
 
 // Tasks i < cnt of one (orbital pair class, auxiliary class) product,
@@ -267,119 +200,24 @@ __global__ void k_scatter_metric(const ScatterM* __restrict__ d, int ntask, cons
   }
 }
 
-// A[Q][m][i] -> At[m][Q][i] (rank x n x o to n x rank x o).
-__global__ void k_permute_qmi(const double* __restrict__ A, double* __restrict__ At, int rank, int n, int o) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t tot = (size_t)rank * n * o;
-  if (idx >= tot) return;
-  const int i = (int)(idx % o);
-  const size_t r = idx / o;
-  const int m = (int)(r % n);
-  const int q = (int)(r / n);
-  At[((size_t)m * rank + q) * o + i] = A[idx];
-}
-
 __global__ void k_axpby_fock(const double* H, const double* J, const double* K, double* F, size_t nn) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nn) F[i] = H[i] + J[i] - 0.5 * K[i];
 }
-
-// Precision conversions for DF-K on the matrix cores.
-__global__ void k_to_f32(const double* __restrict__ x, float* __restrict__ y, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    y[i] = (float)x[i];
-}
-// x = hi + lo with hi = bf16(x) and lo = bf16(x - hi) (round to nearest): the
-// pair carries about 16 significant bits.
-template <class T>
-__global__ void k_split_bf16(const T* __restrict__ x, __hip_bfloat16* __restrict__ hi, __hip_bfloat16* __restrict__ lo,
-                             size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const float v = (float)x[i];
-    const __hip_bfloat16 h = __float2bfloat16(v);
-    hi[i] = h;
-    lo[i] = __float2bfloat16(v - __bfloat162float(h));
-  }
-}
-__global__ void k_f32_to_f64_scaled(const float* __restrict__ x, double* __restrict__ y, size_t n, double s) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    y[i] = s * (double)x[i];
-}
-// A[Q][m][i] -> At[m][Q][i] for float data.
-__global__ void k_permute_qmi_f32(const float* __restrict__ A, float* __restrict__ At, int rank, int n, int o) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t tot = (size_t)rank * n * o;
-  if (idx >= tot) return;
-  const int i = (int)(idx % o);
-  const int m = (int)((idx / o) % n);
-  const int q = (int)(idx / ((size_t)o * n));
-  At[((size_t)m * rank + q) * o + i] = A[idx];
-}
-
-// K = 2 sum_b part[b] over the split-K partial products.
-template <class T>
-__global__ void k_sum_parts(const T* __restrict__ part, int nb, size_t nn, double* __restrict__ K) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (size_t)gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += (double)part[(size_t)b * nn + i];
-    K[i] = 2.0 * s;
-  }
-}
-
-// df_mfma.hip: K = alpha X X^T, and A = B C from the packed factor, on the
-// FP64 matrix cores.
-void syrk_f64(const double* X, int n, long long L, long long ldx, double alpha, double* K, DevBuf& scratch,
-              hipStream_t st);
-void bc_packed_f64(const double* Bp, size_t np, int rank, int n, const double* C, int o, double* At,
-                   long long ldt, double alpha, double* gamma, DevBuf& scratch, hipStream_t st);
-void bc_packed_bf16x3(const double* Bp, size_t np, int rank, int n, const double* C, int o, unsigned short* Ah,
-                      unsigned short* Al, long long ldt, DevBuf& ct, hipStream_t st);
 
 struct DfEngine {
   hipStream_t stream = nullptr;
   std::unique_ptr<Blas> bl;
   int n = 0, naux = 0, rank = 0;
   std::vector<Shell> orb, aux;
-  // B: rank x n x n, or rank x n(n+1)/2 packed (columns ij = i(i+1)/2 + j,
-  // i >= j) when the unpacked 3-index tensor and B would not fit in HBM
-  bool packed = false;
-  size_t npk = 0;
+  size_t npt = 0;  // doubles of one row of the tiled B
   DevBuf d_B;
-  DevBuf d_pk, d_unp;  // packed path: packed P and J; unpacked rows of B for DF-K
-  DevBuf d_syrk;       // partial tiles of the hand-written exchange product
-  DevBuf d_bcp;        // tile partials of B_Q . P from the packed A = B C
-  DevBuf d_ct;         // split BF16 C^T of the packed split-BF16 A = B C
-  // FP64 exchange product by the hand-written MFMA kernel (HFG_DF_SYRK=0: rocBLAS dgemm)
-  const bool use_syrk = [] {
-    const char* e = std::getenv("HFG_DF_SYRK");
-    return !(e && std::atoi(e) == 0);
-  }();
-  // packed factor, FP64 and split BF16: A = B C by the hand-written kernels
-  // straight from the packed rows (HFG_DF_BCPACK=0: unpacked chunks and
-  // rocBLAS GEMMs)
-  // d = B P by k_rowdot (HFG_DF_ROWDOT=0: rocBLAS dgemv)
-  const bool use_rowdot = [] {
-    const char* e = std::getenv("HFG_DF_ROWDOT");
-    return !(e && std::atoi(e) == 0);
-  }();
-  const bool use_bcpack = [] {
-    const char* e = std::getenv("HFG_DF_BCPACK");
-    return !(e && std::atoi(e) == 0);
-  }();
-  DevBuf d_work, d_A, d_At;
-  size_t work_o = 0;
-  // reduced-precision copies of B (made on first use) and work arrays
-  DevBuf d_B32, d_Bh, d_Bl, d_C32, d_Ch, d_Cl, d_A32, d_At32, d_Ah, d_Al, d_K32, d_parts;
-  size_t work_o32 = 0;
-  // Split-K of the reduced-precision K = 2 At At^T (n x n output, inner
-  // dimension rank*o): the output alone gives too few tiles for the chip, so
-  // the auxiliary index is cut into nsplit blocks computed as one strided
-  // batch, then summed in FP64.
-  static constexpr size_t T_CHUNK = 8ull << 30;  // bytes of one column chunk of the packed 3-index tensor
-  int nsplit() const {
-    const int tiles = std::max(1, ((n + 127) / 128) * ((n + 127) / 128));
-    return std::max(1, std::min(rank, (1024 + tiles - 1) / tiles));
-  }
+  // kept between calls: P, its tiled form and the tiled J, d = B P, and the
+  // exchange products' workspace
+  DevBuf d_P, d_tj, d_q;
+  DevBuf d_io;  // J, K and C of a call with host buffers
+  ExchangeWork xwork;
+  static constexpr size_t T_CHUNK = 8ull << 30;  // bytes of one column chunk of the 3-index tensor
 
   DfEngine(const hfg_basis_view& basis, const hfg_basis_view& auxv, double cutoff) {
     if (!(cutoff > 0) || !std::isfinite(cutoff))
@@ -388,21 +226,19 @@ struct DfEngine {
     aux = group_shells(auxv);
     n = basis.n_functions;
     naux = auxv.n_functions;
-    npk = (size_t)n * (n + 1) / 2;
+    npt = tiled_size(n);
     for (auto& s : orb)
       if (s.L > 3) throw HfgError{HFG_UNSUPPORTED, "density fitting compiled for orbital shells up to f"};
     for (auto& s : aux)
       if (s.L > 4) throw HfgError{HFG_UNSUPPORTED, "density fitting compiled for auxiliary shells up to g"};
-    // HBM footprint: unpacked, the 3-index tensor and B at naux n^2 doubles
-    // each; packed, B at naux n(n+1)/2 and the tensor one column chunk at a
-    // time (T_CHUNK bytes), so that config-size bases fit.
+    // HBM footprint: B at naux n(n+1)/2 doubles (and the padding of its last
+    // tile row), and the 3-index tensor one chunk at a time.  Where twice
+    // naux n^2 doubles fit easily so do these; beyond, they are checked.
     size_t free_b = 0, total_b = 0;
     HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
     const double metric = 8.0 * 2.0 * (double)naux * naux;
-    const double unpacked = 8.0 * 2.0 * (double)naux * n * n + metric;
-    const char* force = std::getenv("HFG_DF_PACKED");
-    packed = force ? std::atoi(force) != 0 : unpacked > 0.4 * (double)free_b;
-    if (packed && 8.0 * (double)naux * npk + (double)T_CHUNK + metric > 0.8 * (double)free_b)
+    const double half = 8.0 * (double)naux * ((double)n * (n + 1) / 2);
+    if (4.0 * half + metric > 0.4 * (double)free_b && half + (double)T_CHUNK + metric > 0.8 * (double)free_b)
       throw HfgError{HFG_DEVICE, "DF factor B does not fit in the free device memory"};
     HIP_CHECK(hipStreamCreate(&stream));
     bl.reset(new Blas(stream));
@@ -414,6 +250,7 @@ struct DfEngine {
   DfEngine(const hfg_basis_view& basis, double threshold, double budget, CholeskyInfo& info) {
     orb = group_shells(basis);
     n = basis.n_functions;
+    npt = tiled_size(n);
     for (auto& s : orb)
       if (s.L > 2) throw HfgError{HFG_UNSUPPORTED, "Cholesky factors compiled for orbital shells up to d"};
     HIP_CHECK(hipStreamCreate(&stream));
@@ -583,32 +420,23 @@ struct DfEngine {
     HIP_CHECK(hipMemcpyAsync(d_Xt.p, Xt.data(), Xt.size() * 8, hipMemcpyHostToDevice, stream));
     d_V.free();
 
-    // 3-index tensor T[P][mu][nu]: every orbital pair against every
-    // auxiliary shell (src/df.rs:60-78), one (pair class, auxiliary class)
-    // product at a time, in batches of at most `budget` block doubles, then
-    // B = X^T T.  Packed, the tensor is formed one chunk of function rows
-    // [f0, f1) at a time -- its packed columns f0(f0+1)/2 .. f1(f1+1)/2 - 1,
-    // the pairs whose later shell starts in the chunk -- and each chunk's
-    // columns of B follow from one GEMM, so the tensor never exists whole.
-    const size_t nn = (size_t)n * n;
-    std::vector<std::pair<int, int>> rows;  // function-row chunks
-    if (!packed) {
-      rows.push_back({0, n});
-    } else {
-      std::vector<int> starts;
-      for (auto& sh : orb) starts.push_back(sh.ao);
-      std::sort(starts.begin(), starts.end());
-      starts.push_back(n);
-      auto cols_of = [](long long f0, long long f1) { return f1 * (f1 + 1) / 2 - f0 * (f0 + 1) / 2; };
-      size_t k = 0;
-      while (k + 1 < starts.size()) {
-        size_t e = k + 1;
-        while (e + 1 < starts.size() && 8.0 * naux * cols_of(starts[k], starts[e + 1]) <= (double)T_CHUNK) ++e;
-        rows.push_back({starts[k], starts[e]});
-        k = e;
-      }
+    // 3-index tensor (P|mu nu): every orbital pair against every auxiliary
+    // shell (src/df.rs:60-78), one (pair class, auxiliary class) product at a
+    // time, in batches of at most `budget` block doubles, then B = X^T T.  The
+    // tensor is formed one chunk of tile rows [I0, I1) at a time -- the tiles
+    // I0(I0+1)/2 .. I1(I1+1)/2 - 1 of every row -- and each chunk's columns of B
+    // follow from one GEMM, so the tensor never exists whole.  A shell pair
+    // whose functions lie in two chunks is evaluated for both.
+    const int nt = tiles_of(n);
+    auto tiles_before = [](int I) { return (size_t)I * (I + 1) / 2; };
+    std::vector<std::pair<int, int>> rows;  // chunks of tile rows
+    for (int I = 0; I < nt;) {
+      int e = I + 1;
+      while (e < nt && 8.0 * naux * (tiles_before(e + 1) - tiles_before(I)) * (TL * TL) <= (double)T_CHUNK) ++e;
+      rows.push_back({I, e});
+      I = e;
     }
-    d_B.alloc((size_t)rank * (packed ? npk : nn) * 8);
+    d_B.alloc((size_t)rank * npt * 8);
     DevBuf d_T;
     std::map<int, std::vector<int>> by_xc;  // auxiliary class -> shells
     for (int p = 0; p < (int)aux.size(); ++p) by_xc[pair_class(aux[p].L, 0)].push_back(p);
@@ -616,14 +444,16 @@ struct DfEngine {
     DevBuf d_opair, d_oa, d_ob, d_xsh, d_xao, dt, ds3, dout;
     size_t cap_tasks = 0, cap_out = 0;
     for (const auto& rc : rows) {
-      const long long c0 = (long long)rc.first * (rc.first + 1) / 2;
-      const long long cols = packed ? (long long)rc.second * (rc.second + 1) / 2 - c0 : (long long)nn;
+      const size_t c0 = tiles_before(rc.first) * (TL * TL), cols = tiles_before(rc.second) * (TL * TL) - c0;
       const size_t tsz = (size_t)naux * cols;
       if (d_T.bytes < tsz * 8) d_T.alloc(tsz * 8);
-      std::map<int, std::vector<int>> by_oc;  // orbital pair class -> pairs of this chunk
+      hipLaunchKernelGGL(k_zero, dim3((unsigned)((tsz + 255) / 256)), dim3(256), 0, stream, d_T.as<double>(), tsz);
+      std::map<int, std::vector<int>> by_oc;  // orbital pair class -> pairs with functions in this chunk
       for (int i = 0; i < norb_pairs; ++i) {
-        const int row = std::max(pairs[i].ao_a, pairs[i].ao_b);
-        if (row >= rc.first && row < rc.second) by_oc[pair_class(pairs[i].la, pairs[i].lb)].push_back(i);
+        const PairInfo& pr = pairs[i];
+        const int la = pr.ao_a + nc(pr.la) - 1, lb = pr.ao_b + nc(pr.lb) - 1;  // last functions
+        if (std::max(la, lb) / TL >= rc.first && std::max(pr.ao_a, pr.ao_b) / TL < rc.second)
+          by_oc[pair_class(pr.la, pr.lb)].push_back(i);
       }
       for (auto& oc : by_oc) {
         const std::vector<int>& ol = oc.second;
@@ -674,12 +504,8 @@ struct DfEngine {
               launch_block_class(cls, args, stream);
             else  // an orbital f-p, f-d or f-f pair (never on the auxiliary side)
               launch_df_f_block(o0.la, o0.lb, aux[xl[0]].L, 0, args, stream);
-            if (packed)
-              hipLaunchKernelGGL(k_scatter3p, dim3(cnt), dim3(64), 0, stream, ds3.as<Scatter3>(), cnt,
-                                 dout.as<double>(), d_so.as<double>(), d_sx.as<double>(), d_T.as<double>(), c0, cols);
-            else
-              hipLaunchKernelGGL(k_scatter3, dim3(cnt), dim3(64), 0, stream, ds3.as<Scatter3>(), cnt,
-                                 dout.as<double>(), d_so.as<double>(), d_sx.as<double>(), d_T.as<double>(), n);
+            hipLaunchKernelGGL(k_scatter3, dim3(cnt), dim3(64), 0, stream, ds3.as<Scatter3>(), cnt, dout.as<double>(),
+                               d_so.as<double>(), d_sx.as<double>(), d_T.as<double>(), rc.first, rc.second, c0, cols);
             HIP_CHECK(hipGetLastError());
           }
           // the lists are rewritten for the next product
@@ -687,221 +513,42 @@ struct DfEngine {
         }
       }
       // B[:, chunk] = X^T T_chunk  (rank x naux) (naux x cols)
-      const int ldb = (int)(packed ? npk : nn);
       bl->gemm(false, false, rank, (int)cols, naux, 1.0, d_Xt.as<double>(), naux, d_T.as<double>(), (int)cols, 0.0,
-               d_B.as<double>() + (packed ? c0 : 0), ldb);
+               d_B.as<double>() + c0, (int)npt);
       HIP_CHECK(hipStreamSynchronize(stream));
     }
   }
 
-  // Packed B: f(q0, qn, W, lo) for chunks of rows q0 .. q0+qn-1 unpacked to
-  // qn symmetric n x n matrices W of type T (for BF16, W the high and lo the
-  // low part of the split), about 2 GB of scratch at a time.
-  template <class T, class F>
-  void for_unpacked_rows(F&& f) {
-    const size_t nn = (size_t)n * n;
-    const int qc = (int)std::max<size_t>(1, std::min<size_t>(rank, (2ull << 30) / (nn * 8)));
-    if (d_unp.bytes < (size_t)qc * nn * 8) d_unp.alloc((size_t)qc * nn * 8);
-    T* W = d_unp.as<T>();
-    __hip_bfloat16* lo = std::is_same<T, __hip_bfloat16>::value ? d_unp.as<__hip_bfloat16>() + (size_t)qc * nn
-                                                                 : nullptr;
-    for (int q0 = 0; q0 < rank; q0 += qc) {
-      const int qn = std::min(qc, rank - q0);
-      const int nt = (n + 63) / 64;
-      hipLaunchKernelGGL(k_unpack_tiles<T>, dim3((unsigned)(nt * (nt + 1) / 2), (unsigned)qn), dim3(256), 0, stream,
-                         d_B.as<double>() + (size_t)q0 * npk, n, npk, nt, W, lo);
-      HIP_CHECK(hipGetLastError());
-      f(q0, qn, (const T*)W, (const __hip_bfloat16*)lo);
-    }
-  }
-
   // J = sum_Q B_Q (B_Q . P), P = 2 C C^T; K = 2 sum_Q (B_Q C)(B_Q C)^T
-  // (src/df.rs:143-173).  dC: n x o device; outputs device n x n.
-  void jk(const double* dC, int o, double* dJ, double* dK) {
+  // (src/df.rs:143-173), the exchange in the given precision (df_mfma.hip), J in
+  // FP64.  dC: n x o device; outputs device n x n.  FP64 exchange gives
+  // B_Q . P = 2 sum A_Q . C from its tiles; otherwise it is a pass over B.
+  void jk(const double* dC, int o, double* dJ, double* dK, int precision) {
     const size_t nn = (size_t)n * n;
-    // packed factor with K: A = B C by the packed kernel straight into the
-    // exchange layout, B P taken from its tiles (B_Q . P = 2 sum A_Q . C)
-    const bool fused = packed && use_bcpack && dK;
-    if ((size_t)o != work_o) {
-      d_work.alloc(std::max(nn, (size_t)rank) * 8 + 8);
-      d_A.free();
-      d_At.alloc((size_t)rank * n * o * 8);
-      work_o = o;
+    if (!d_q.p) {
+      d_q.alloc((size_t)rank * 8);
+      d_tj.alloc(2 * npt * 8);
     }
-    if (dK && !fused && d_A.bytes < (size_t)rank * n * o * 8) d_A.alloc((size_t)rank * n * o * 8);
-    double* P = d_work.as<double>();
-    Dev dq;
-    dq.alloc(rank);
-    bl->gemm(false, true, n, n, o, 2.0, dC, o, dC, o, 0.0, P, n);
-    const double one = 1.0, zero = 0.0;
-    const size_t bc = packed ? npk : nn;  // columns of B
-    const double* pv = P;
-    double* jv = dJ;
-    if (packed) {
-      // packed P with the off-diagonal doubled, so that B P over the packed
-      // columns is the full contraction; J comes back packed
-      if (d_pk.bytes < 2 * npk * 8) d_pk.alloc(2 * npk * 8);
-      hipLaunchKernelGGL(k_pack_sym2, dim3((unsigned)((npk + 255) / 256)), dim3(256), 0, stream, P, n,
-                         d_pk.as<double>());
+    double* dq = d_q.as<double>();
+    double* tiled_p = d_tj.as<double>();
+    double* tiled_j = tiled_p + npt;
+    if (precision == 0) {
+      df_exchange(d_B.as<double>(), npt, rank, n, dC, o, 0, dK, dq, xwork, stream);
+    } else {
+      if (!d_P.p) d_P.alloc(nn * 8);
+      double* P = d_P.as<double>();
+      bl->gemm(false, true, n, n, o, 2.0, dC, o, dC, o, 0.0, P, n);
+      hipLaunchKernelGGL(k_tile_sym2, dim3((unsigned)((npt + 255) / 256)), dim3(256), 0, stream, P, n, npt, tiled_p);
       HIP_CHECK(hipGetLastError());
-      pv = d_pk.as<double>();
-      jv = d_pk.as<double>() + npk;
-    }
-    // column-major view of B: bc x rank (B^T); d = B P  ->  gemv(T)
-    if (fused)
-      bc_packed_f64(d_B.as<double>(), npk, rank, n, dC, o, d_At.as<double>(), (long long)rank * o, 2.0, dq.p, d_bcp,
-                    stream);
-    else if (use_rowdot) {
       hipLaunchKernelGGL(k_rowdot, dim3((unsigned)((rank + RD_ROWS - 1) / RD_ROWS)), dim3(RD_NT), 0, stream,
-                         d_B.as<double>(), bc, bc, rank, pv, dq.p);
+                         d_B.as<double>(), npt, npt, rank, tiled_p, dq);
       HIP_CHECK(hipGetLastError());
-    } else
-      RB_CHECK(rocblas_dgemv(bl->h, rocblas_operation_transpose, (rocblas_int)bc, rank, &one, d_B.as<double>(),
-                             (rocblas_int)bc, pv, 1, &zero, dq.p, 1));
-    RB_CHECK(rocblas_dgemv(bl->h, rocblas_operation_none, (rocblas_int)bc, rank, &one, d_B.as<double>(),
-                           (rocblas_int)bc, dq.p, 1, &zero, jv, 1));
-    if (packed) {
-      hipLaunchKernelGGL(k_unpack_sym, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, stream, jv, n, dJ);
-      HIP_CHECK(hipGetLastError());
+      df_exchange(d_B.as<double>(), npt, rank, n, dC, o, precision, dK, nullptr, xwork, stream);
     }
-    if (!dK) return;  // J only
-    if (!fused) {
-      // A = B C: rows (Q, m), (rank*n) x o, then permuted to At[m][Q o + i]
-      if (!packed)
-        bl->gemm(false, false, rank * n, o, n, 1.0, d_B.as<double>(), n, dC, o, 0.0, d_A.as<double>(), o);
-      else
-        for_unpacked_rows<double>([&](int q0, int qn, const double* W, const __hip_bfloat16*) {
-          bl->gemm(false, false, qn * n, o, n, 1.0, W, n, dC, o, 0.0, d_A.as<double>() + (size_t)q0 * n * o, o);
-        });
-      const size_t tot = (size_t)rank * n * o;
-      hipLaunchKernelGGL(k_permute_qmi, dim3((tot + 255) / 256), dim3(256), 0, stream, d_A.as<double>(),
-                         d_At.as<double>(), rank, n, o);
-      HIP_CHECK(hipGetLastError());
-    }
-    // FP64: the symmetric product on the matrix cores (upper tiles only,
-    // split over the contraction index); or one rocBLAS GEMM (its dsyrk,
-    // with half the flops, ran 2.1x slower than the GEMM on (H2O)32/cc-pVDZ)
-    if (use_syrk)
-      syrk_f64(d_At.as<double>(), n, (long long)rank * o, (long long)rank * o, 2.0, dK, d_syrk, stream);
-    else
-      bl->gemm(false, true, n, n, rank * o, 2.0, d_At.as<double>(), rank * o, d_At.as<double>(), rank * o, 0.0, dK,
-               n);
-  }
-
-  // DF-K in reduced precision on the matrix cores (J stays FP64, HBM-bound):
-  // prec 1: FP32 operands, FP32 accumulation; prec 2: each operand split into
-  // two BF16 parts, three BF16 products (hi*hi + hi*lo + lo*hi) with FP32
-  // accumulation, for both A = B C and K = 2 At At^T.  No reference
-  // counterpart: the reference's DF-K is FP64 (src/df.rs:143-173).
-  void gemm_ex(bool ta, bool tb, int m, int nn_, int k, const void* A, int lda, const void* B, int ldb, float* C,
-               int ldc, float alpha, float beta, rocblas_datatype in) {
-    // row-major C = op(A) op(B) through column-major C^T = op(B)^T op(A)^T
-    RB_CHECK(rocblas_gemm_ex(bl->h, tb ? rocblas_operation_transpose : rocblas_operation_none,
-                             ta ? rocblas_operation_transpose : rocblas_operation_none, nn_, m, k, &alpha, B, in, ldb,
-                             A, in, lda, &beta, C, rocblas_datatype_f32_r, ldc, C, rocblas_datatype_f32_r, ldc,
-                             rocblas_datatype_f32_r, rocblas_gemm_algo_standard, 0, 0));
-  }
-  void k_reduced(const double* dC, int o, double* dK, int prec) {
-    const size_t nn = (size_t)n * n, bsz = (size_t)rank * nn, csz = (size_t)n * o, asz = (size_t)rank * n * o;
-    const dim3 g(2048), b(256);
-    if (prec == 1 && !packed && !d_B32.p) {
-      d_B32.alloc(bsz * 4);
-      hipLaunchKernelGGL(k_to_f32, g, b, 0, stream, d_B.as<double>(), d_B32.as<float>(), bsz);
-    }
-    if (prec == 2 && !packed && !d_Bh.p) {
-      d_Bh.alloc(bsz * 2);
-      d_Bl.alloc(bsz * 2);
-      hipLaunchKernelGGL(k_split_bf16<double>, g, b, 0, stream, d_B.as<double>(), d_Bh.as<__hip_bfloat16>(),
-                         d_Bl.as<__hip_bfloat16>(), bsz);
-    }
-    // packed factor, split BF16: the hi and lo operands of the symmetric
-    // product straight from the packed rows (no unpack, FP32 A or permute)
-    const bool direct = prec == 2 && packed && use_bcpack;
-    if ((size_t)o != work_o32) {
-      d_C32.alloc(csz * 4);
-      d_Ch.alloc(csz * 2);
-      d_Cl.alloc(csz * 2);
-      d_A32.free();
-      d_At32.free();
-      d_Ah.alloc(asz * 2);
-      d_Al.alloc(asz * 2);
-      d_K32.alloc(nn * 4);
-      work_o32 = o;
-    }
-    if (!direct && !d_A32.p) {
-      d_A32.alloc(asz * 4);
-      d_At32.alloc(asz * 4);
-    }
-    float* A = d_A32.as<float>();
-    float* At = d_At32.as<float>();
-    float* K = d_K32.as<float>();
-    if (direct) {
-      bc_packed_bf16x3(d_B.as<double>(), npk, rank, n, dC, o, (unsigned short*)d_Ah.p, (unsigned short*)d_Al.p,
-                       (long long)rank * o, d_ct, stream);
-    } else if (prec == 1) {
-      hipLaunchKernelGGL(k_to_f32, g, b, 0, stream, dC, d_C32.as<float>(), csz);
-      if (!packed)
-        gemm_ex(false, false, rank * n, o, n, d_B32.p, n, d_C32.p, o, A, o, 1.f, 0.f, rocblas_datatype_f32_r);
-      else
-        for_unpacked_rows<float>([&](int q0, int qn, const float* W, const __hip_bfloat16*) {
-          gemm_ex(false, false, qn * n, o, n, W, n, d_C32.p, o, A + (size_t)q0 * n * o, o, 1.f, 0.f,
-                  rocblas_datatype_f32_r);
-        });
-    } else {
-      hipLaunchKernelGGL(k_split_bf16<double>, g, b, 0, stream, dC, d_Ch.as<__hip_bfloat16>(),
-                         d_Cl.as<__hip_bfloat16>(), csz);
-      const auto bf = rocblas_datatype_bf16_r;
-      auto three = [&](const void* Bh, const void* Bl, int rows, float* Ao) {
-        gemm_ex(false, false, rows, o, n, Bh, n, d_Ch.p, o, Ao, o, 1.f, 0.f, bf);
-        gemm_ex(false, false, rows, o, n, Bh, n, d_Cl.p, o, Ao, o, 1.f, 1.f, bf);
-        gemm_ex(false, false, rows, o, n, Bl, n, d_Ch.p, o, Ao, o, 1.f, 1.f, bf);
-      };
-      if (!packed)
-        three(d_Bh.p, d_Bl.p, rank * n, A);
-      else
-        for_unpacked_rows<__hip_bfloat16>([&](int q0, int qn, const __hip_bfloat16* Wh, const __hip_bfloat16* Wl) {
-          three(Wh, Wl, qn * n, A + (size_t)q0 * n * o);
-        });
-    }
-    if (!direct)
-      hipLaunchKernelGGL(k_permute_qmi_f32, dim3((asz + 255) / 256), dim3(256), 0, stream, A, At, rank, n, o);
-    (void)K;
-    const int nb = nsplit(), qb = (rank + nb - 1) / nb, nbe = (rank + qb - 1) / qb, full = rank / qb;
-    const int kc = qb * o, ld = rank * o;
-    d_parts.alloc((size_t)nbe * nn * 4);
-    float* parts = d_parts.as<float>();
-    // partial[b] (+)= X_b Y_b^T over aux block b, X, Y the row-major n x (rank*o)
-    // operands; column-major: partial^T = Y_b^T-ish, same as gemm_ex above.
-    auto split_gemm = [&](const void* X, const void* Y, float beta, rocblas_datatype in, size_t esz) {
-      const float one = 1.f;
-      if (full > 0)
-        RB_CHECK(rocblas_gemm_strided_batched_ex(bl->h, rocblas_operation_transpose, rocblas_operation_none, n, n, kc,
-                                                 &one, Y, in, ld, kc, X, in, ld, kc, &beta, parts,
-                                                 rocblas_datatype_f32_r, n, (rocblas_stride)nn, parts,
-                                                 rocblas_datatype_f32_r, n, (rocblas_stride)nn, full,
-                                                 rocblas_datatype_f32_r, rocblas_gemm_algo_standard, 0, 0));
-      if (full < nbe) {
-        const int kt = (rank - full * qb) * o;
-        const char* Xt = (const char*)X + (size_t)full * kc * esz;
-        const char* Yt = (const char*)Y + (size_t)full * kc * esz;
-        RB_CHECK(rocblas_gemm_ex(bl->h, rocblas_operation_transpose, rocblas_operation_none, n, n, kt, &one, Yt, in,
-                                 ld, Xt, in, ld, &beta, parts + (size_t)full * nn, rocblas_datatype_f32_r, n,
-                                 parts + (size_t)full * nn, rocblas_datatype_f32_r, n, rocblas_datatype_f32_r,
-                                 rocblas_gemm_algo_standard, 0, 0));
-      }
-    };
-    if (prec == 1) {
-      split_gemm(At, At, 0.f, rocblas_datatype_f32_r, 4);
-    } else {
-      if (!direct)
-        hipLaunchKernelGGL(k_split_bf16<float>, g, b, 0, stream, At, d_Ah.as<__hip_bfloat16>(),
-                           d_Al.as<__hip_bfloat16>(), asz);
-      const auto bf = rocblas_datatype_bf16_r;
-      split_gemm(d_Ah.p, d_Ah.p, 0.f, bf, 2);
-      split_gemm(d_Ah.p, d_Al.p, 1.f, bf, 2);
-      split_gemm(d_Al.p, d_Ah.p, 1.f, bf, 2);
-    }
-    hipLaunchKernelGGL(k_sum_parts<float>, dim3(1024), dim3(256), 0, stream, parts, nbe, nn, dK);
+    const double one = 1.0, zero = 0.0;  // column-major view of B: npt x rank
+    RB_CHECK(rocblas_dgemv(bl->h, rocblas_operation_none, (rocblas_int)npt, rank, &one, d_B.as<double>(),
+                           (rocblas_int)npt, dq, 1, &zero, tiled_j, 1));
+    hipLaunchKernelGGL(k_untile_sym, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, stream, tiled_j, n, dJ);
     HIP_CHECK(hipGetLastError());
   }
 };
@@ -994,13 +641,8 @@ static int df_rhf(const hfg_basis_view* basis, const std::function<DfEngine*()>&
   int fp64_builds = 0;
   auto fock = [&](double* F) {
     const auto tf = clk::now();
-    if (kprec != 0) {
-      df.jk(dCo.p, no, dJ.p, nullptr);  // J in FP64
-      df.k_reduced(dCo.p, no, dK.p, kprec);
-    } else {
-      df.jk(dCo.p, no, dJ.p, dK.p);
-      ++fp64_builds;
-    }
+    df.jk(dCo.p, no, dJ.p, dK.p, kprec);
+    if (kprec == 0) ++fp64_builds;
     hipLaunchKernelGGL(k_axpby_fock, grid(nn), dim3(tb), 0, st, dH.p, dJ.p, dK.p, F, nn);
     HIP_CHECK(hipStreamSynchronize(st));
     t_fock += std::chrono::duration<double>(clk::now() - tf).count();
@@ -1122,6 +764,47 @@ struct hfg_df {
   std::unique_ptr<DfEngine> e;
 };
 
+// J and K of host coefficients into host buffers, through the handle's staging
+// buffer; device_ms (may be null): device time of the contraction.
+static int df_host_jk(hfg_df* df, const double* cocc, int nocc, double* j, double* k, int precision,
+                      double* device_ms) {
+  if (!df || !cocc || !j || !k || nocc <= 0) return dferr(HFG_INVALID_INPUT, "invalid occupied coefficients for DF J/K");
+  if (precision < 0 || precision > 2) return dferr(HFG_INVALID_INPUT, "precision must be 0 (FP64), 1 (FP32) or 2 (BF16x3)");
+  try {
+    DfEngine& e = *df->e;
+    const size_t nn = (size_t)e.n * e.n, no = (size_t)e.n * nocc;
+    for (size_t x = 0; x < no; ++x)
+      if (!std::isfinite(cocc[x])) return dferr(HFG_INVALID_INPUT, "invalid occupied coefficients for DF J/K");
+    if (e.d_io.bytes < (2 * nn + no) * 8) e.d_io.alloc((2 * nn + no) * 8);
+    double *dj = e.d_io.as<double>(), *dk = dj + nn, *dc = dk + nn;
+    upload(dc, cocc, no, e.stream);
+    hipEvent_t ev[2] = {};
+    struct Events {
+      hipEvent_t* ev;
+      ~Events() {
+        for (int x = 0; x < 2; ++x)
+          if (ev[x]) (void)hipEventDestroy(ev[x]);
+      }
+    } events{ev};
+    if (device_ms) {
+      for (hipEvent_t& x : ev) HIP_CHECK(hipEventCreate(&x));
+      HIP_CHECK(hipEventRecord(ev[0], e.stream));
+    }
+    e.jk(dc, nocc, dj, dk, precision);
+    if (device_ms) HIP_CHECK(hipEventRecord(ev[1], e.stream));
+    download(j, dj, nn, e.stream);
+    download(k, dk, nn, e.stream);
+    if (device_ms) {
+      float ms = 0;
+      HIP_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
+      *device_ms = ms;
+    }
+    return HFG_OK;
+  } catch (HfgError& ex) {
+    return dferr(ex.code, ex.msg);
+  }
+}
+
 extern "C" {
 
 int hfg_df_build(const hfg_basis_view* basis, const hfg_basis_view* aux, double metric_cutoff, hfg_df** out) {
@@ -1154,67 +837,12 @@ int hfg_df_info(const hfg_df* df, int64_t* n, int64_t* naux, int64_t* rank) {
 }
 
 int hfg_df_jk(hfg_df* df, const double* cocc, int nocc, double* j, double* k) {
-  if (!df || !cocc || !j || !k || nocc <= 0) return dferr(HFG_INVALID_INPUT, "invalid occupied coefficients for DF J/K");
-  try {
-    DfEngine& e = *df->e;
-    const size_t nn = (size_t)e.n * e.n;
-    for (size_t x = 0; x < (size_t)e.n * nocc; ++x)
-      if (!std::isfinite(cocc[x])) return dferr(HFG_INVALID_INPUT, "invalid occupied coefficients for DF J/K");
-    Dev dc, dj, dk;
-    dc.alloc((size_t)e.n * nocc);
-    dj.alloc(nn);
-    dk.alloc(nn);
-    upload(dc.p, cocc, (size_t)e.n * nocc, e.stream);
-    e.jk(dc.p, nocc, dj.p, dk.p);
-    download(j, dj.p, nn, e.stream);
-    download(k, dk.p, nn, e.stream);
-    return HFG_OK;
-  } catch (HfgError& ex) {
-    return dferr(ex.code, ex.msg);
-  }
+  return df_host_jk(df, cocc, nocc, j, k, 0, nullptr);
 }
 
 int hfg_df_jk_ex(hfg_df* df, const double* cocc, int nocc, double* j, double* k, int precision,
                  double* device_ms) {
-  if (!df || !cocc || !j || !k || nocc <= 0) return dferr(HFG_INVALID_INPUT, "invalid occupied coefficients for DF J/K");
-  if (precision < 0 || precision > 2) return dferr(HFG_INVALID_INPUT, "precision must be 0 (FP64), 1 (FP32) or 2 (BF16x3)");
-  try {
-    DfEngine& e = *df->e;
-    const size_t nn = (size_t)e.n * e.n;
-    for (size_t x = 0; x < (size_t)e.n * nocc; ++x)
-      if (!std::isfinite(cocc[x])) return dferr(HFG_INVALID_INPUT, "invalid occupied coefficients for DF J/K");
-    Dev dc, dj, dk;
-    dc.alloc((size_t)e.n * nocc);
-    dj.alloc(nn);
-    dk.alloc(nn);
-    upload(dc.p, cocc, (size_t)e.n * nocc, e.stream);
-    if (precision != 0) {  // first use: make the reduced copies of B outside the timed region
-      e.k_reduced(dc.p, nocc, dk.p, precision);
-      HIP_CHECK(hipStreamSynchronize(e.stream));
-    }
-    hipEvent_t e0, e1;
-    HIP_CHECK(hipEventCreate(&e0));
-    HIP_CHECK(hipEventCreate(&e1));
-    HIP_CHECK(hipEventRecord(e0, e.stream));
-    if (precision == 0) {
-      e.jk(dc.p, nocc, dj.p, dk.p);
-    } else {
-      e.jk(dc.p, nocc, dj.p, nullptr);  // J in FP64
-      e.k_reduced(dc.p, nocc, dk.p, precision);
-    }
-    HIP_CHECK(hipEventRecord(e1, e.stream));
-    HIP_CHECK(hipEventSynchronize(e1));
-    float ms = 0;
-    HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (device_ms) *device_ms = ms;
-    download(j, dj.p, nn, e.stream);
-    download(k, dk.p, nn, e.stream);
-    return HFG_OK;
-  } catch (HfgError& ex) {
-    return dferr(ex.code, ex.msg);
-  }
+  return df_host_jk(df, cocc, nocc, j, k, precision, device_ms);
 }
 
 int hfg_df_rhf(const hfg_basis_view* basis, const hfg_basis_view* aux, const double* zxyz, int natom, int charge,

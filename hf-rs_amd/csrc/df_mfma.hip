@@ -1,553 +1,313 @@
-// df_mfma.hip -- the exchange product of DF-K, K = alpha X X^T (X: n x L,
-// row-major, L = rank * n_occ), on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64): coulomb_exchange_rhf's K += 2 A_Q A_Q^T summed
-// over Q (src/df.rs:143-173) as one symmetric rank-L update.
+// df_mfma.hip -- the exchange products of DF-K on the matrix cores, straight
+// from the tiled factor: A_Q = B_Q C for every auxiliary row Q, and
+// K = 2 sum_Q A_Q A_Q^T = 2 X X^T (coulomb_exchange_rhf's loop over Q,
+// src/df.rs:143-173, as one symmetric rank-L update with L = rank n_occ), in
+// FP64, in FP32 and with operands split into two BF16 parts.
 //
-// Only the tiles on and above the diagonal are computed (half the FLOPs of a
-// GEMM).  Each 256-thread workgroup takes one 128 x 128 output tile and one
-// slice of the contraction index: the tiles alone are far too few for 256
-// CUs (28 at n = 800), so L is cut into S slices whose partial tiles go to a
-// buffer [S][n][n] and are summed in a fixed order by a second kernel, which
-// also writes the lower triangle.  Per 16-wide step of the contraction the
-// two 128 x 16 panels of X are staged in LDS (rows padded to 17 doubles: the
-// 16 rows one MFMA operand reads fall in distinct banks), the next step's
-// panels are loaded into registers meanwhile; each wave owns a 64 x 64
-// quarter of the tile, sixteen 16 x 16 accumulators.
+// The tiled factor (df_tiles.h): row Q holds the lower triangle of B_Q in
+// 32 x 32 tiles.  Both kernels work on panels of 16-byte chunks: a panel row
+// is one matrix row (or column) of a contraction step, CH chunks of 16 bytes
+// (2 FP64, 4 FP32 or 8 BF16 values), and a lane's operand is one chunk, read
+// from LDS with one 16-byte load: in a group of MFMAs lane l takes row l % 16
+// and the chunk of its lane group l / 16, so that FP64 and FP32 chunks feed
+// two and four consecutive MFMAs (the order of the contraction index within
+// a step is free as long as both operands share it).  Chunks are stored at
+// c ^ swz(row), which spreads the 16 rows that one operand reads over all LDS
+// banks without padding.
 //
-// MFMA f64 16x16x4 operand layout (lane l): A[i][k] with i = l % 16,
-// k = l / 16; B[k][j] with j = l % 16, k = l / 16; D[i][j] in register r of
-// lane l with j = l % 16, i = l / 16 + 4 r (rows interleaved by register,
-// unlike the 4-row groups of the FP32 16x16x4 form).
+// MFMA layouts (lane l): operand row or column l % 16, contraction index from
+// l / 16; the FP64 16x16x4 result has column l % 16 and row l / 16 + 4 r in
+// register r, the FP32 and BF16 16x16 forms row 4 (l / 16) + r.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
-#include <vector>
+#include <type_traits>
 
+#include "df_tiles.h"
 #include "engine.h"
 
 namespace hfg {
 namespace {
 
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
 
-constexpr int ST = 128;     // output tile
-constexpr int KB = 32;      // contraction step staged in LDS
-constexpr int PAD = KB + 1;
-constexpr int SYRK_NT = 512;  // 8 waves, 4 x 2 over the tile
-constexpr int WTI = ST / 4, WTJ = ST / 2;  // a wave's rows and columns of the tile
-constexpr int NBI = WTI / 16, NBJ = WTJ / 16;  // 16 x 16 MFMA blocks per wave side
+template <class To, class From>
+__device__ __forceinline__ To as_bits(From x) {
+  static_assert(sizeof(To) == sizeof(From), "same size");
+  return __builtin_bit_cast(To, x);
+}
 
-// The thread's share of the two ST x KB panels at contraction offset k0:
-// row t / 4, columns 8 (t % 4) .. +7 of each (zero beyond n rows or kend).
-struct Panel {
-  double a[8], b[8];
+// FP32 pair -> BF16 pair (round to nearest even) and back
+__device__ __forceinline__ unsigned bf16_pair(f2 v) { return as_bits<unsigned>(__builtin_convertvector(v, b2)); }
+__device__ __forceinline__ f2 bf16_values(unsigned p) {
+  return f2{__uint_as_float(p << 16), __uint_as_float(p & 0xffff0000u)};
+}
+
+// The three arithmetics.  CH: 16-byte chunks of a panel row of the A = B C
+// step (32 contraction values); acc: accumulator of one 16 x 16 block; X: an
+// element of the exchange product's operand; XK: contraction values in its
+// 256-byte step; P: a partial sum; SUB: MFMAs of a chunk pair.
+struct F64 {
+  static constexpr int CH = 16, XK = 32, SUB = 2;
+  typedef d4 acc;
+  typedef double X, P;
+  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
 };
-__device__ __forceinline__ void load_panel(const double* __restrict__ X, int n, long long ldx, int i0, int j0,
-                                           long long k0, long long kend, bool vec, Panel& p) {
-  const int t = threadIdx.x, r = t >> 2, c0 = (t & 3) * 8;
-  const int ra = i0 + r, rb = j0 + r;
-  const long long k = k0 + c0;
-  if (vec && k + 8 <= kend) {
-    // 16-byte loads: rows start 16-byte aligned when ldx is even, k0 is a multiple of KB
+struct F32 {
+  static constexpr int CH = 8, XK = 64, SUB = 4;
+  typedef f4 acc;
+  typedef float X, P;
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+// x = hi + lo, hi = bf16(x), lo = bf16(x - hi); hi hi + hi lo + lo hi summed in
+// FP32.  Panel rows hold the hi chunks, then the lo chunks; the exchange
+// operand alternates 64 hi and the same 64 lo values.
+struct BF16x3 {
+  static constexpr int CH = 8, XK = 64, SUB = 3;
+  typedef f4 acc;
+  typedef unsigned short X;
+  typedef float P;
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+template <int CH>
+__device__ __forceinline__ int swz(int row) {
+  return CH == 16 ? row & 15 : (row >> 1) & 7;
+}
+
+// Sub-step s of one chunk pair: FP64 and FP32 take one value of each chunk, BF16
+// one of the products hi hi, hi lo, lo hi.
+__device__ __forceinline__ void mac(F64, int s, d4& acc, u4 a, u4, u4 b, u4) {
+  acc = __builtin_amdgcn_mfma_f64_16x16x4f64(as_bits<d2>(a)[s], as_bits<d2>(b)[s], acc, 0, 0, 0);
+}
+__device__ __forceinline__ void mac(F32, int s, f4& acc, u4 a, u4, u4 b, u4) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(as_bits<f4>(a)[s], as_bits<f4>(b)[s], acc, 0, 0, 0);
+}
+__device__ __forceinline__ void mac(BF16x3, int s, f4& acc, u4 ah, u4 al, u4 bh, u4 bl) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bits<b8>(s == 2 ? al : ah), as_bits<b8>(s == 1 ? bl : bh), acc, 0,
+                                                0, 0);
+}
+
+// A 256-thread workgroup's four waves over a tile of 64 rows and NB 16-column
+// blocks: 2 x 2 waves of 32 rows and NB / 2 blocks (7 chunks read for 10 chunk
+// products at NB = 10), 4 x 1 of 16 rows where NB is odd.
+template <int NB>
+struct Waves {
+  static constexpr int M = NB % 2 ? 4 : 2, N = 4 / M, RA = 4 / M, NBW = NB / N;
+};
+constexpr int ROWS = 64, NT = 256;
+
+// One step over LDS panels of CHP chunks a row (rows of A at ra + 16 x, columns
+// of B at cb + 16 b): the chunks of the step, or for BF16 the hi chunks of its
+// first half with the lo chunks of its second.
+template <class T, int CHP, int RA, int NBW>
+__device__ __forceinline__ void step(typename T::acc (&acc)[RA][NBW], const u4* A, const u4* B, int ra, int cb,
+                                     int lane) {
+  const int rq = lane & 15, g = lane >> 4;
+  constexpr bool BF = T::SUB == 3;
+  constexpr int GROUPS = BF ? CHP / 8 : CHP / 4;  // groups of four chunks (BF16: of hi chunks)
 #pragma unroll
-    for (int c = 0; c < 8; c += 2) {
-      const double2 va = ra < n ? *(const double2*)(X + (size_t)ra * ldx + k + c) : double2{0.0, 0.0};
-      const double2 vb = rb < n ? *(const double2*)(X + (size_t)rb * ldx + k + c) : double2{0.0, 0.0};
-      p.a[c] = va.x;
-      p.a[c + 1] = va.y;
-      p.b[c] = vb.x;
-      p.b[c + 1] = vb.y;
-    }
-  } else {
+  for (int t = 0; t < GROUPS; ++t) {
+    u4 a[RA], al[RA], v[NBW], vl[NBW];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const bool kin = k + c < kend;
-      p.a[c] = (ra < n && kin) ? X[(size_t)ra * ldx + k + c] : 0.0;
-      p.b[c] = (rb < n && kin) ? X[(size_t)rb * ldx + k + c] : 0.0;
+    for (int x = 0; x < RA; ++x) {
+      const int r = ra + 16 * x + rq;
+      a[x] = A[r * CHP + ((4 * t + g) ^ swz<CHP>(r))];
+      al[x] = BF ? A[r * CHP + ((CHP / 2 + 4 * t + g) ^ swz<CHP>(r))] : a[x];
     }
+#pragma unroll
+    for (int b = 0; b < NBW; ++b) {
+      const int r = cb + 16 * b + rq;
+      v[b] = B[r * CHP + ((4 * t + g) ^ swz<CHP>(r))];
+      vl[b] = BF ? B[r * CHP + ((CHP / 2 + 4 * t + g) ^ swz<CHP>(r))] : v[b];
+    }
+#pragma unroll
+    for (int s = 0; s < T::SUB; ++s)
+#pragma unroll
+      for (int b = 0; b < NBW; ++b)
+#pragma unroll
+        for (int x = 0; x < RA; ++x) mac(T(), s, acc[x][b], a[x], al[x], v[b], vl[b]);
   }
 }
 
-__global__ __launch_bounds__(SYRK_NT) void k_syrk_f64(const double* __restrict__ X, int n, long long L,
-                                                      long long ldx, const int2* __restrict__ tiles, int ntile,
-                                                      long long kslice, double* __restrict__ part) {
-  __shared__ double As[2][ST * PAD], Bs[2][ST * PAD];
-  const int2 tile = tiles[blockIdx.x % ntile];
-  const int s = blockIdx.x / ntile;
-  const int i0 = tile.x * ST, j0 = tile.y * ST;
-  const long long kbeg = (long long)s * kslice, kend = L < kbeg + kslice ? L : kbeg + kslice;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wi = w >> 1, wj = w & 1;
-  const bool vec = (ldx & 1) == 0;
-  d4 acc[NBI][NBJ];
+// ---- A = B C
+
+// The pair kp of a panel row's 32 values (FP64 2 kp, 2 kp + 1) -> LDS.
+__device__ __forceinline__ void put2(F64, u4* L, int r, int kp, d2 v) { L[r * 16 + (kp ^ swz<16>(r))] = as_bits<u4>(v); }
+__device__ __forceinline__ void put2(F32, u4* L, int r, int kp, d2 v) {
+  ((f2*)(L + r * 8 + ((kp >> 1) ^ swz<8>(r))))[kp & 1] = f2{(float)v.x, (float)v.y};
+}
+__device__ __forceinline__ void split2(d2 v, unsigned& h, unsigned& l) {
+  const f2 x = {(float)v.x, (float)v.y};
+  h = bf16_pair(x);
+  const f2 y = bf16_values(h);
+  l = bf16_pair(f2{x.x - y.x, x.y - y.y});
+}
+__device__ __forceinline__ void put2(BF16x3, u4* L, int r, int kp, d2 v) {
+  unsigned h, l;
+  split2(v, h, l);
+  ((unsigned*)(L + r * 8 + ((kp >> 2) ^ swz<8>(r))))[kp & 3] = h;
+  ((unsigned*)(L + r * 8 + ((4 + (kp >> 2)) ^ swz<8>(r))))[kp & 3] = l;
+}
+
+// C (n x o, FP64) -> panels [column tile it][k tile kb][column < an][CH chunks],
+// zero past (n, o): what one workgroup's step reads is one contiguous run.
+template <class T>
+__global__ __launch_bounds__(256) void k_pack_c(const double* __restrict__ C, int n, int o, int nt, int an, int gy,
+                                                u4* __restrict__ out) {
+  const int e = blockIdx.x * 256 + threadIdx.x;  // (it, kb, pair of values, column)
+  if (e >= gy * nt * an * 16) return;
+  const int col = e % an, kp = (e / an) & 15, rest = e / an / 16;
+  const int k = rest % nt * TL + 2 * kp, i = (rest / nt) * an + col;
+  d2 v = {0.0, 0.0};
+  if (i < o) {
+    if (k < n) v.x = C[(size_t)k * o + i];
+    if (k + 1 < n) v.y = C[(size_t)(k + 1) * o + i];
+  }
+  u4* row = out + (size_t)(rest * an + col) * T::CH;
+  if constexpr (T::CH == 16) {
+    row[kp] = as_bits<u4>(v);
+  } else if constexpr (T::SUB == 4) {
+    ((f2*)row)[kp] = f2{(float)v.x, (float)v.y};
+  } else {
+    unsigned h, l;
+    split2(v, h, l);
+    ((unsigned*)row)[kp] = h;
+    ((unsigned*)row)[16 + kp] = l;
+  }
+}
+
+// The exchange operand X (n x L, contraction index k = Q o + i) is stored step by
+// step: the n rows' 256 bytes of a step are one run, so that what a workgroup
+// reads of a step, and what it writes of a row Q, lies in a few pages.  (Row by
+// row, with rows of 5 MB, every panel row was in a page of its own.)
+__device__ __forceinline__ void put_x(double* X, int n, int m, long long k, double v) {
+  X[((k >> 5) * n + m) * 32 + (k & 31)] = v;
+}
+__device__ __forceinline__ void put_x(float* X, int n, int m, long long k, float v) {
+  X[((k >> 6) * n + m) * 64 + (k & 63)] = v;
+}
+__device__ __forceinline__ void put_x(unsigned short* X, int n, int m, long long k, float v) {
+  const unsigned h = bf16_pair(f2{v, 0.f}) & 0xffffu;
+  const unsigned l = bf16_pair(f2{v - __uint_as_float(h << 16), 0.f}) & 0xffffu;
+  unsigned short* p = X + ((k >> 6) * n + m) * 128 + (k & 63);
+  p[0] = (unsigned short)h;
+  p[64] = (unsigned short)l;
+}
+
+// A workgroup takes two 32-row blocks -- consecutive (Q, tile row I) pairs, so
+// that no row is padding beyond the last tile of a row Q -- against NB x 16
+// columns of C.  Step kb multiplies tile (I, kb) of each block, read along its
+// rows where kb <= I and as the transpose of tile (kb, I) above the diagonal,
+// with the C panel of that tile column.  A block is staged by a pair of waves as
+// pairs of consecutive contraction values, converted (and split) once: along
+// its rows, one 16-byte load of 64 consecutive pairs a wave; as a transpose,
+// two 8-byte loads along two of its rows.
+// One LDS buffer and two barriers a step, the next step's panels on their way
+// to registers meanwhile: half the LDS of a second buffer lets two workgroups
+// share a CU, and while one stages, the other multiplies.  (One 512-thread
+// workgroup of 128 rows and two buffers: the two waves of a SIMD move in step
+// and the matrix cores idle while both wait, 75 % busy.)
+// Output: X[m][Q o + i] (put_x), and with part the sums of A_Q . C over each
+// wave's rows of a block (B_Q . P without another pass over B).
+// Workgroups are dealt round-robin to the 8 XCDs by linear id; id 8 j + x takes
+// item off(x) + j, so that each XCD runs a contiguous run of blocks and the
+// two reads of a tile (as itself and transposed) meet in its L2.
+template <class T, int NB>
+__global__ __launch_bounds__(NT) void k_bc_tiles(const double* __restrict__ Bt, size_t npt, int nt, int rank, int n,
+                                                 const u4* __restrict__ Cp, const double* __restrict__ C, int o,
+                                                 typename T::X* __restrict__ X, double* __restrict__ part, int gy,
+                                                 int total) {
+  typedef Waves<NB> W;
+  constexpr int CH = T::CH, AN = 16 * NB, RA = W::RA, NBW = W::NBW;
+  constexpr int NC = (AN * CH + NT - 1) / NT;  // C chunks a thread stages
+  __shared__ u4 lds[(ROWS + AN) * CH];
+  u4* lc = lds + ROWS * CH;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int per = total / 8, rem = total % 8, xcd = blockIdx.x % 8;
+  const int item = xcd * per + min(xcd, rem) + blockIdx.x / 8;
+  const int it = item % gy;
+  const int nblk = rank * nt;
+  const int f0 = (item / gy) * 2;
+  // the block this thread stages, by pairs of waves
+  const int fs = min(f0 + (w >> 1), nblk - 1);
+  const int qs = fs / nt, is = fs - qs * nt;
+  const double* Bq = Bt + (size_t)qs * npt;
+  const int h = w & 1;
+  constexpr bool even = AN * CH % NT == 0;
+  d2 bv[4];
+  u4 cv[NC];
+  auto load = [&](int kb) {
+    const double* tile = Bq + tile_index(is, kb) * (TL * TL);
+    if (kb <= is) {
 #pragma unroll
-  for (int a = 0; a < NBI; ++a)
+      for (int c = 0; c < 4; ++c) bv[c] = ((const d2*)tile)[256 * h + 64 * c + lane];
+    } else {
+      const double* p = tile + (16 * h + 2 * (lane >> 5)) * TL + (lane & 31);
 #pragma unroll
-    for (int b = 0; b < NBJ; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
-  const int r = t >> 2, c0 = (t & 3) * 8;
-  auto store = [&](const Panel& p, int buf) {
+      for (int c = 0; c < 4; ++c) {
+        bv[c].x = p[4 * c * TL];
+        bv[c].y = p[(4 * c + 1) * TL];
+      }
+    }
+    const u4* cp = Cp + ((size_t)it * nt + kb) * AN * CH;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      As[buf][r * PAD + c0 + c] = p.a[c];
-      Bs[buf][r * PAD + c0 + c] = p.b[c];
+    for (int c = 0; c < NC; ++c)
+      if (even || t + NT * c < AN * CH) cv[c] = cp[NT * c + t];
+  };
+  auto store = [&](int kb) {
+    const bool low = kb <= is;
+    const int r = 32 * (w >> 1) + (low ? 16 * h + (lane >> 4) : lane & 31), kp = low ? lane & 15 : 8 * h + (lane >> 5);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) put2(T(), lds, low ? r + 4 * c : r, low ? kp : kp + 2 * c, bv[c]);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int e = t + NT * c, col = e / CH;
+      if (even || e < AN * CH) lc[col * CH + ((e % CH) ^ swz<CH>(col))] = cv[c];
     }
   };
-  // buffer cur holds the step's panels, the registers the next step's; a step
-  // stores them into the other buffer (whose readers all passed the previous
-  // barrier), loads the step after, multiplies, and meets the other waves at
-  // one barrier
-  Panel nxt;
-  if (kbeg < kend) {
-    load_panel(X, n, ldx, i0, j0, kbeg, kend, vec, nxt);
-    store(nxt, 0);
-    if (kbeg + KB < kend) load_panel(X, n, ldx, i0, j0, kbeg + KB, kend, vec, nxt);
-  }
-  __syncthreads();
-  int cur = 0;
-  for (long long k0 = kbeg; k0 < kend; k0 += KB, cur ^= 1) {
-    if (k0 + KB < kend) {
-      store(nxt, cur ^ 1);
-      if (k0 + 2 * KB < kend) load_panel(X, n, ldx, i0, j0, k0 + 2 * KB, kend, vec, nxt);
-    }
-    const double* as = As[cur];
-    const double* bs = Bs[cur];
-#pragma unroll
-    for (int kk = 0; kk < KB; kk += 4) {
-      const int kq = kk + (lane >> 4), rq = lane & 15;
-      double av[NBI], bv[NBJ];
-#pragma unroll
-      for (int a = 0; a < NBI; ++a) av[a] = as[(WTI * wi + 16 * a + rq) * PAD + kq];
-#pragma unroll
-      for (int b = 0; b < NBJ; ++b) bv[b] = bs[(WTJ * wj + 16 * b + rq) * PAD + kq];
-#pragma unroll
-      for (int a = 0; a < NBI; ++a)
-#pragma unroll
-        for (int b = 0; b < NBJ; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-    }
+  typename T::acc acc[RA][NBW] = {};
+  const int wm = w % W::M, wn = w / W::M;
+  load(0);
+  for (int kb = 0; kb < nt; ++kb) {
+    if (kb) __syncthreads();  // every wave has read the last step's panels
+    store(kb);
+    if (kb + 1 < nt) load(kb + 1);
     __syncthreads();
+    step<T, CH>(acc, lds, lc, 16 * RA * wm, 16 * NBW * wn, lane);
   }
-  double* out = part + (size_t)s * n * n;
-#pragma unroll
-  for (int a = 0; a < NBI; ++a)
-#pragma unroll
-    for (int b = 0; b < NBJ; ++b)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int i = i0 + WTI * wi + 16 * a + (lane >> 4) + 4 * q;
-        const int j = j0 + WTJ * wj + 16 * b + (lane & 15);
-        if (i < n && j < n) out[(size_t)i * n + j] = acc[a][b][q];
-      }
-}
-
-// K[i][j] = alpha sum_s part[s][tile-upper position of (i, j)], both triangles.
-__global__ void k_syrk_reduce(const double* __restrict__ part, int nslice, int n, double alpha,
-                              double* __restrict__ K) {
-  const size_t nn = (size_t)n * n;
-  for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < nn; idx += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(idx / n), j = (int)(idx - (size_t)i * n);
-    const size_t src = (i / ST <= j / ST) ? idx : (size_t)j * n + i;
-    double v = 0.0;
-    for (int s = 0; s < nslice; ++s) v += part[(size_t)s * nn + src];
-    K[idx] = alpha * v;
-  }
-}
-
-// ---- Work order of the packed A = B C kernels.  Each packed element of B_Q
-// is read by two workgroups: the one of its row's 128-row tile and, as the
-// transposed element, the one of its column's tile.  Two choices make the
-// second read a cache hit:
-// - XCD-aware mapping: workgroups are dealt round-robin to the 8 XCDs by
-//   linear id, so linear id L = 8 j + x is given work item off(x) + j: each
-//   XCD takes a contiguous run of items, the tiles of one auxiliary row run
-//   together on one XCD and share its L2;
-// - tournament order over the k-tiles (the circle method on M = T or T + 1
-//   players, M odd, plus a fixed player F = M): in round r tile i multiplies
-//   k-tile (2 r - i) mod M and the tile named there multiplies k-tile i, so
-//   both reads of a 128 x 128 packed block fall in the same round; tile i
-//   meets F in round i and takes its diagonal block then, a round against
-//   the padding player (T even) is skipped.
-// Measured on (H2O)32 / cc-pVTZ (ms a launch, neither / XCD map / tournament
-// / both): FP64 111.8 / 111.3 / 119.6 / 119.2, split BF16 52.9 / 47.3 / 44.3
-// / 43.3.  The split-BF16 kernel, bound by the traffic of B, takes both; the
-// FP64 kernel, bound by the matrix cores, only the XCD map.
-constexpr int BC_XCD_MAP = 1, BC_TOURNAMENT = 2;
-struct WorkItem {
-  int mt, it, q;
-};
-__device__ __forceinline__ WorkItem work_item(int gx, int gy, long long total, int flags) {
-  const long long L = blockIdx.x, per = total / 8, rem = total % 8;
-  const int x = (int)(L % 8);
-  const long long w = (flags & BC_XCD_MAP) ? x * per + (x < rem ? x : rem) + L / 8 : L;
-  WorkItem r;
-  r.mt = (int)(w % gx);
-  const long long rest = w / gx;
-  r.it = (int)(rest % gy);
-  r.q = (int)(rest / gy);
-  return r;
-}
-
-template <int KS>
-struct PanelOrder {
-  static constexpr int TS = 128, PPT = TS / KS;  // tile width, panels a tile
-  int mt, T, M, n, tour;
-  __device__ PanelOrder(int mt_, int n_, int flags)
-      : mt(mt_), T((n_ + TS - 1) / TS), M(T | 1), n(n_), tour(flags & BC_TOURNAMENT) {}
-  __device__ int count() const { return tour ? M * PPT : (n + KS - 1) / KS; }
-  // k0 of panel s (tournament: s = r PPT + j), or -1 where there is none
-  __device__ int k0(int s) const {
-    if (!tour) return s * KS;
-    const int r = s / PPT, j = s - r * PPT;
-    int t = r == mt ? mt : ((2 * r - mt) % M + M) % M;
-    if (t >= T) return -1;
-    const int k = t * TS + j * KS;
-    return k < n ? k : -1;
-  }
-  __device__ int next(int s) const {
-    for (++s; s < count(); ++s)
-      if (k0(s) >= 0) break;
-    return s;
-  }
-};
-
-// A_Q = B_Q C for every row Q of the packed factor
-// (B_Q symmetric n x n, lower triangle row-major, packed row stride np; C
-// n x o row-major), written as At[m][Q o + i] (the exchange product's
-// operand, row stride ldt), and with part, the tile's sum of A_Q . C
-// (B_Q . P for P = C C^T without another pass over B).  One workgroup of NT
-// threads per 128 x 160 tile of A_Q, in the work order above (all 160 columns of a 160-orbital C in one tile,
-// so that B is read once).  Per 16-wide contraction step the B panel comes
-// from the packed rows -- along packed row k where the panel lies above the
-// diagonal (k > every m of the tile), along packed row m below it, by
-// (max, min) where the diagonal crosses it -- consecutive lanes reading
-// consecutive doubles; the next panel is loaded into registers while the
-// current one is multiplied out of the other LDS buffer, one barrier a step.
-// Waves (NT / 128) x 2, each 128 / (NT / 128) rows x 80 columns of 16 x 16
-// MFMA blocks.
-constexpr int AM = 128, AN = 160, AK = 32;
-static_assert(AM == PanelOrder<AK>::TS, "tiles of the panel order are the row tiles");
-constexpr int APB = AK + 1, APC = AN + 1;
-
-template <int NT>
-struct BcRegs {
-  static constexpr int LR = NT / AK;         // lanes along a panel row
-  static constexpr int NB = AM * AK / NT;    // B values per thread
-  static constexpr int NC = AN * AK / NT;    // C values per thread
-  double b[NB], c[NC];
-};
-
-template <int NT>
-__device__ __forceinline__ void bc_load(const double* __restrict__ B, int n, const double* __restrict__ C, int o,
-                                        int m0, int i0, int k0, int t, BcRegs<NT>& r) {
-  constexpr int LR = BcRegs<NT>::LR, NB = BcRegs<NT>::NB, NC = BcRegs<NT>::NC;
-  if (k0 >= m0 + AM) {
-    const int k = k0 + t / LR;
-    const size_t base = (size_t)k * (k + 1) / 2;
-#pragma unroll
-    for (int c = 0; c < NB; ++c) {
-      const int m = m0 + t % LR + LR * c;
-      r.b[c] = (k < n && m < n) ? B[base + m] : 0.0;
-    }
-  } else if (k0 + AK <= m0) {
-    const int k = k0 + t % AK;
-#pragma unroll
-    for (int c = 0; c < NB; ++c) {
-      const int m = m0 + t / AK + LR * c;
-      r.b[c] = (k < n && m < n) ? B[(size_t)m * (m + 1) / 2 + k] : 0.0;
-    }
-  } else {
-    const int k = k0 + t % AK;
-#pragma unroll
-    for (int c = 0; c < NB; ++c) {
-      const int m = m0 + t / AK + LR * c;
-      const size_t hi = m > k ? m : k, lo = m > k ? k : m;
-      r.b[c] = (k < n && m < n) ? B[hi * (hi + 1) / 2 + lo] : 0.0;
-    }
-  }
-  const int k = k0 + t / LR;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int i = i0 + t % LR + LR * c;
-    r.c[c] = (k < n && i < o) ? C[(size_t)k * o + i] : 0.0;
-  }
-}
-
-template <int NT>
-__device__ __forceinline__ void bc_store(int m0, int k0, int t, const BcRegs<NT>& r, double* Bs, double* Cs) {
-  constexpr int LR = BcRegs<NT>::LR, NB = BcRegs<NT>::NB, NC = BcRegs<NT>::NC;
-  if (k0 >= m0 + AM) {
-#pragma unroll
-    for (int c = 0; c < NB; ++c) Bs[(t % LR + LR * c) * APB + t / LR] = r.b[c];
-  } else {
-#pragma unroll
-    for (int c = 0; c < NB; ++c) Bs[(t / AK + LR * c) * APB + t % AK] = r.b[c];
-  }
-#pragma unroll
-  for (int c = 0; c < NC; ++c) Cs[(t / LR) * APC + t % LR + LR * c] = r.c[c];
-}
-
-template <int NT>
-__global__ __launch_bounds__(NT) void k_bc_packed_f64(const double* __restrict__ Bp, size_t np, int n,
-                                                      const double* __restrict__ C, int o,
-                                                      double* __restrict__ At, long long ldt,
-                                                      double* __restrict__ part, int gx, int gy, long long total, int flags) {
-  constexpr int WR = AM / (NT / 128), BA = WR / 16;  // rows per wave, MFMA blocks along them
-  __shared__ double Bs[2][AM * APB], Cs[2][AK * APC];
-  const WorkItem wi = work_item(gx, gy, total, flags);
-  const int m0 = wi.mt * AM, i0 = wi.it * AN, q = wi.q;
-  const double* B = Bp + (size_t)q * np;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  d4 acc[BA][5];
-#pragma unroll
-  for (int a = 0; a < BA; ++a)
-#pragma unroll
-    for (int b = 0; b < 5; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
-  // Panels in tournament order: panel s in buffer cur, the registers hold
-  // panel s1.  A step stores the registers into the other buffer (whose
-  // readers all passed the previous barrier), loads panel s2, multiplies, and
-  // meets the other waves at one barrier.
-  const PanelOrder<AK> po(wi.mt, n, flags);
-  const int S = po.count();
-  int s = po.next(-1), s1 = po.next(s);
-  BcRegs<NT> r;
-  bc_load<NT>(B, n, C, o, m0, i0, po.k0(s), t, r);
-  bc_store<NT>(m0, po.k0(s), t, r, Bs[0], Cs[0]);
-  if (s1 < S) bc_load<NT>(B, n, C, o, m0, i0, po.k0(s1), t, r);
-  __syncthreads();
-  for (int cur = 0; s < S; cur ^= 1) {
-    const int s2 = s1 < S ? po.next(s1) : S;
-    if (s1 < S) {
-      bc_store<NT>(m0, po.k0(s1), t, r, Bs[cur ^ 1], Cs[cur ^ 1]);
-      if (s2 < S) bc_load<NT>(B, n, C, o, m0, i0, po.k0(s2), t, r);
-    }
-    const double* bs = Bs[cur];
-    const double* cs = Cs[cur];
-#pragma unroll
-    for (int kk = 0; kk < AK; kk += 4) {
-      const int kq = kk + (lane >> 4), rq = lane & 15;
-      double av[BA], bv[5];
-#pragma unroll
-      for (int a = 0; a < BA; ++a) av[a] = bs[(WR * wm + 16 * a + rq) * APB + kq];
-#pragma unroll
-      for (int b = 0; b < 5; ++b) bv[b] = cs[kq * APC + 80 * wn + 16 * b + rq];
-#pragma unroll
-      for (int a = 0; a < BA; ++a)
-#pragma unroll
-        for (int b = 0; b < 5; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();
-    s = s1;
-    s1 = s2;
-  }
-  // A_Q[m][i] -> At[m][Q o + i]; with part, this tile's sum of A_Q . C
-  double* Aq = At + (size_t)q * o;
+  // a wave's rows lie in one block
+  const int fb = f0 + 16 * RA * wm / 32;
+  if (fb >= nblk) return;
+  const int q = fb / nt, m0 = (fb - q * nt) * TL + 16 * RA * wm % 32;
   double sum = 0.0;
 #pragma unroll
-  for (int a = 0; a < BA; ++a)
+  for (int a = 0; a < RA; ++a)
 #pragma unroll
-    for (int b = 0; b < 5; ++b)
+    for (int b = 0; b < NBW; ++b)
 #pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int m = m0 + WR * wm + 16 * a + (lane >> 4) + 4 * x;
-        const int i = i0 + 80 * wn + 16 * b + (lane & 15);
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + 16 * a + T::row(lane, r), i = it * AN + 16 * (NBW * wn + b) + (lane & 15);
         if (m < n && i < o) {
-          Aq[(size_t)m * ldt + i] = acc[a][b][x];
-          if (part) sum += acc[a][b][x] * C[(size_t)m * o + i];
+          put_x(X, n, m, (long long)q * o + i, acc[a][b][r]);
+          if (part) sum += (double)acc[a][b][r] * C[(size_t)m * o + i];
         }
       }
-  if (part) {  // fixed-order block sum
-    __shared__ double red[NT];
-    red[t] = sum;
-    __syncthreads();
-    for (int h = NT / 2; h > 0; h >>= 1) {
-      if (t < h) red[t] += red[t + h];
-      __syncthreads();
-    }
-    if (t == 0) part[(size_t)q * gx * gy + wi.it * gx + wi.mt] = red[0];
+  if (part) {  // two waves to a block: two halves of its rows, or of the columns
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) sum += __shfl_xor(sum, s, 64);
+    if (lane == 0) part[((size_t)fb * gy + it) * 2 + (RA == 2 ? wn : wm & 1)] = sum;
   }
 }
 
-// ---- split-BF16 form: A = B C with each operand x = hi + lo (hi = bf16(x),
-// lo = bf16(x - hi), from the FP32 value) and three BF16 products hi hi +
-// hi lo + lo hi accumulated in FP32, then A itself split into the hi and lo
-// BF16 operands of the symmetric product.
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-
-// FP32 -> BF16 bits, round to nearest even (finite values), as __float2bfloat16
-__device__ __forceinline__ unsigned bf16_bits(float f) {
-  const unsigned u = __float_as_uint(f);
-  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-}
-__device__ __forceinline__ float bf16_value(unsigned h) { return __uint_as_float(h << 16); }
-__device__ __forceinline__ void split_bf16(float f, unsigned& h, unsigned& l) {
-  h = bf16_bits(f);
-  l = bf16_bits(f - bf16_value(h));
-}
-
-constexpr int SM = 128, SN = 160, SK = 32, SP = 40;  // tile rows, columns, contraction step, LDS row (BF16)
-static_assert(SM == PanelOrder<SK>::TS, "tiles of the panel order are the row tiles");
-constexpr int SBUF = (2 * SM + 2 * SN) * SP;         // BF16 per LDS buffer: B hi, B lo, C hi, C lo
-
-// C (n x o, FP64) -> hi and lo parts of C^T, [oc][nk] BF16, zero past (o, n)
-__global__ void k_split_ct(const double* __restrict__ C, int n, int o, int nk, int oc, unsigned short* __restrict__ Th,
-                           unsigned short* __restrict__ Tl) {
-  const size_t tot = (size_t)oc * nk;
-  for (size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x; x < tot; x += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(x / nk), k = (int)(x - (size_t)i * nk);
-    unsigned h = 0, l = 0;
-    if (i < o && k < n) split_bf16((float)C[(size_t)k * o + i], h, l);
-    Th[x] = (unsigned short)h;
-    Tl[x] = (unsigned short)l;
-  }
-}
-
-struct SplitRegs {
-  double b[8];       // B[m][k0 + 8 g + c], c < 8
-  uint4 ch[2], cl[2];  // 8 BF16 of C^T rows (chunks t and t + 512 of the 640)
-};
-
-__device__ __forceinline__ bool split_above(int m0, int k0) { return k0 >= m0 + SM; }
-
-__device__ __forceinline__ void split_load(const double* __restrict__ B, int n, const unsigned short* __restrict__ Th,
-                                           const unsigned short* __restrict__ Tl, int nk, int m0, int i0, int k0,
-                                           int t, SplitRegs& r) {
-  if (split_above(m0, k0)) {  // packed row k, consecutive m across lanes
-    const int m = m0 + (t & 127), g = t >> 7;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int k = k0 + 8 * g + c;
-      r.b[c] = (k < n && m < n) ? B[(size_t)k * (k + 1) / 2 + m] : 0.0;
-    }
-  } else if (k0 + SK <= m0) {  // packed row m, consecutive k
-    const int m = m0 + (t >> 2), g = t & 3;
-    const size_t base = (size_t)m * (m + 1) / 2;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int k = k0 + 8 * g + c;
-      r.b[c] = (k < n && m < n) ? B[base + k] : 0.0;
-    }
-  } else {
-    const int m = m0 + (t >> 2), g = t & 3;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int k = k0 + 8 * g + c;
-      const size_t hi = m > k ? m : k, lo = m > k ? k : m;
-      r.b[c] = (k < n && m < n) ? B[hi * (hi + 1) / 2 + lo] : 0.0;
-    }
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int cid = t + 512 * h;
-    if (h == 0 || t < 128) {
-      const size_t at = (size_t)(i0 + (cid >> 2)) * nk + k0 + 8 * (cid & 3);
-      r.ch[h] = *(const uint4*)(Th + at);
-      r.cl[h] = *(const uint4*)(Tl + at);
-    }
-  }
-}
-
-__device__ __forceinline__ void split_store(int m0, int k0, int t, const SplitRegs& r, unsigned short* S) {
-  unsigned short *Bh = S, *Bl = S + SM * SP, *Ch = S + 2 * SM * SP, *Cl = Ch + SN * SP;
-  const bool above = split_above(m0, k0);
-  const int mm = above ? (t & 127) : (t >> 2), g = above ? (t >> 7) : (t & 3);
-  unsigned h[8], l[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) split_bf16((float)r.b[c], h[c], l[c]);
-  *(uint4*)(Bh + mm * SP + 8 * g) = uint4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
-  *(uint4*)(Bl + mm * SP + 8 * g) = uint4{l[0] | l[1] << 16, l[2] | l[3] << 16, l[4] | l[5] << 16, l[6] | l[7] << 16};
-#pragma unroll
-  for (int x = 0; x < 2; ++x) {
-    const int cid = t + 512 * x;
-    if (x == 0 || t < 128) {
-      *(uint4*)(Ch + (cid >> 2) * SP + 8 * (cid & 3)) = r.ch[x];
-      *(uint4*)(Cl + (cid >> 2) * SP + 8 * (cid & 3)) = r.cl[x];
-    }
-  }
-}
-
-// The split-BF16 A = B C from the packed factor: tiles, panel cases and
-// pipeline as k_bc_packed_f64 (128 x 160 per 512-thread workgroup, waves
-// 4 x 2 of 32 x 80), a 32-wide contraction step per v_mfma_f32_16x16x32_bf16;
-// B split while it is staged, C^T pre-split ([oc][nk], k contiguous, so each
-// lane's 8 contraction values are one 16-byte LDS read for either operand).
-// Output: the hi and lo BF16 parts of A at Ah/Al[m][Q o + i] (row stride ldt).
-__global__ __launch_bounds__(512) void k_bc_packed_bf16x3(const double* __restrict__ Bp, size_t np, int n,
-                                                          const unsigned short* __restrict__ Th,
-                                                          const unsigned short* __restrict__ Tl, int nk, int o,
-                                                          unsigned short* __restrict__ Ah,
-                                                          unsigned short* __restrict__ Al, long long ldt, int gx,
-                                                          int gy, long long total, int flags) {
-  __shared__ uint4 lds[2][SBUF / 8];
-  const WorkItem wi = work_item(gx, gy, total, flags);
-  const int m0 = wi.mt * SM, i0 = wi.it * SN, q = wi.q;
-  const double* B = Bp + (size_t)q * np;
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int wm = w >> 1, wn = w & 1, rq = lane & 15, g = lane >> 4;
-  f4 acc[2][5];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 5; ++b) acc[a][b] = f4{0.f, 0.f, 0.f, 0.f};
-  const PanelOrder<SK> po(wi.mt, n, flags);
-  const int S = po.count();
-  int s = po.next(-1), s1 = po.next(s);
-  SplitRegs r;
-  split_load(B, n, Th, Tl, nk, m0, i0, po.k0(s), t, r);
-  split_store(m0, po.k0(s), t, r, (unsigned short*)lds[0]);
-  if (s1 < S) split_load(B, n, Th, Tl, nk, m0, i0, po.k0(s1), t, r);
-  __syncthreads();
-  for (int cur = 0; s < S; cur ^= 1) {
-    const int s2 = s1 < S ? po.next(s1) : S;
-    if (s1 < S) {
-      split_store(m0, po.k0(s1), t, r, (unsigned short*)lds[cur ^ 1]);
-      if (s2 < S) split_load(B, n, Th, Tl, nk, m0, i0, po.k0(s2), t, r);
-    }
-    const unsigned short* S = (const unsigned short*)lds[cur];
-    const unsigned short *Bh = S, *Bl = S + SM * SP, *Ch = S + 2 * SM * SP, *Cl = Ch + SN * SP;
-    bf8 ah[2], al[2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      ah[a] = *(const bf8*)(Bh + (32 * wm + 16 * a + rq) * SP + 8 * g);
-      al[a] = *(const bf8*)(Bl + (32 * wm + 16 * a + rq) * SP + 8 * g);
-    }
-#pragma unroll
-    for (int b = 0; b < 5; ++b) {
-      const bf8 ch = *(const bf8*)(Ch + (80 * wn + 16 * b + rq) * SP + 8 * g);
-      const bf8 cl = *(const bf8*)(Cl + (80 * wn + 16 * b + rq) * SP + 8 * g);
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[a], ch, acc[a][b], 0, 0, 0);
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[a], cl, acc[a][b], 0, 0, 0);
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[a], ch, acc[a][b], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-    s = s1;
-    s1 = s2;
-  }
-  // D of the FP32 16 x 16 forms: lane l, register x holds row 4 (l / 16) + x, column l % 16
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 5; ++b)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const int m = m0 + 32 * wm + 16 * a + 4 * g + x;
-        const int i = i0 + 80 * wn + 16 * b + rq;
-        if (m < n && i < o) {
-          unsigned h, l;
-          split_bf16(acc[a][b][x], h, l);
-          const size_t at = (size_t)m * ldt + (size_t)q * o + i;
-          Ah[at] = (unsigned short)h;
-          Al[at] = (unsigned short)l;
-        }
-      }
-}
-
-// gamma[Q] = alpha * (sum of the np tile partials of row Q, in order)
+// gamma[Q] = alpha * (the np sums of row Q, in order)
 __global__ void k_part_reduce(const double* __restrict__ part, int np, int rank, double alpha,
                               double* __restrict__ gamma) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -557,90 +317,228 @@ __global__ void k_part_reduce(const double* __restrict__ part, int np, int rank,
   gamma[q] = alpha * s;
 }
 
-}  // namespace
+// Zero the exchange operand's values k in [L, L + w) of its last step.
+template <class X>
+__global__ void k_zero_tail(X* __restrict__ x, int n, long long L, int w) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < w * n) put_x(x, n, e / w, L + e % w, 0);
+}
 
-// A = B C for every row of the packed factor (rank rows of stride np), into
-// the layout of the exchange product: At[m][Q o + i] (row stride ldt >=
-// rank o).  With gamma, also gamma[Q] = alpha sum_{m,i} A_Q[m][i] C[m][i]
-// (= tr(B_Q P) for P = alpha C C^T), reduced in a fixed order through
-// scratch.  On stream st.
-void bc_packed_f64(const double* Bp, size_t np, int rank, int n, const double* C, int o, double* At,
-                   long long ldt, double alpha, double* gamma, DevBuf& scratch, hipStream_t st) {
-  const unsigned gx = (unsigned)((n + AM - 1) / AM), gy = (unsigned)((o + AN - 1) / AN);
-  double* part = nullptr;
-  if (gamma) {
-    const size_t need = (size_t)rank * gx * gy * 8;
-    if (scratch.bytes < need) scratch.alloc(need);
-    part = scratch.as<double>();
+// Column tile of the A = B C kernel: gy tiles of nb 16-column blocks, the
+// least padded width plus one block's worth a tile for what a tile costs
+// beside its columns.
+void column_tiles(int o, int& nb, int& gy) {
+  const int all = (o + 15) / 16;
+  int best = INT32_MAX;
+  for (int g = (all + 9) / 10; g <= (all + 9) / 10 + 2; ++g) {
+    const int b = (all + g - 1) / g;
+    if (g * (b + 1) < best) {
+      best = g * (b + 1);
+      nb = b;
+      gy = g;
+    }
   }
-  const long long total = (long long)gx * gy * rank;
-  if (total > INT32_MAX) throw HfgError{HFG_UNSUPPORTED, "packed A = B C: too many tiles for one launch"};
-  // 512 threads (2 waves a SIMD) measured 5 % faster than 256 (1 wave a SIMD,
-  // 160 accumulator registers) on (H2O)32 / cc-pVTZ
-  hipLaunchKernelGGL(k_bc_packed_f64<512>, dim3((unsigned)total), dim3(512), 0, st, Bp, np, n, C, o, At, ldt, part,
-                     (int)gx, (int)gy, total, BC_XCD_MAP);
-  HIP_CHECK(hipGetLastError());
-  if (gamma) {
-    hipLaunchKernelGGL(k_part_reduce, dim3((unsigned)((rank + 255) / 256)), dim3(256), 0, st, part, (int)(gx * gy),
-                       rank, alpha, gamma);
+}
+
+template <class T, int NB>
+void launch_bc(int nb, const double* Bt, size_t npt, int nt, int rank, int n, const u4* Cp, const double* C, int o,
+               typename T::X* X, double* part, int gy, hipStream_t st) {
+  if constexpr (NB > 0) {
+    if (nb != NB) {
+      launch_bc<T, NB - 1>(nb, Bt, npt, nt, rank, n, Cp, C, o, X, part, gy, st);
+      return;
+    }
+    const long long total = ((long long)rank * nt + 1) / 2 * gy;
+    if (total > INT32_MAX) throw HfgError{HFG_UNSUPPORTED, "tiled A = B C: too many tiles for one launch"};
+    hipLaunchKernelGGL((k_bc_tiles<T, NB>), dim3((unsigned)total), dim3(NT), 0, st, Bt, npt, nt, rank, n, Cp, C, o, X,
+                       part, gy, (int)total);
     HIP_CHECK(hipGetLastError());
   }
 }
 
-// The split-BF16 A = B C from the packed factor (rank rows of stride np),
-// written as the hi and lo BF16 parts Ah/Al[m][Q o + i] (row stride ldt >=
-// rank o); ct holds the split C^T.  On stream st.
-void bc_packed_bf16x3(const double* Bp, size_t np, int rank, int n, const double* C, int o, unsigned short* Ah,
-                      unsigned short* Al, long long ldt, DevBuf& ct, hipStream_t st) {
-  const int nk = (n + SK - 1) / SK * SK, oc = (o + SN - 1) / SN * SN;
-  const size_t tot = (size_t)oc * nk;
-  if (ct.bytes < 2 * tot * 2) ct.alloc(2 * tot * 2);
-  unsigned short* Th = ct.as<unsigned short>();
-  unsigned short* Tl = Th + tot;
-  hipLaunchKernelGGL(k_split_ct, dim3((unsigned)std::min<size_t>(2048, (tot + 255) / 256)), dim3(256), 0, st, C, n, o,
-                     nk, oc, Th, Tl);
+// ---- K = 2 X X^T
+
+// The exchange product's output tiles: 64 rows against the columns from the
+// tile's own first row on (only the upper triangle is computed: 346k of the
+// 320k elements at n = 800, where 128-row tiles of 128 columns took 459k), in
+// the fewest column tiles of at most ten 16-column blocks, all within one block
+// of each other.
+struct SyrkTile {
+  int i0, j0, nb;  // first row, first column, 16-column blocks
+};
+__host__ __device__ inline int syrk_tiles(int n, int r) { return ((n - ROWS * r + 15) / 16 + 9) / 10; }
+__device__ inline SyrkTile syrk_tile(int n, int x) {
+  for (int r = 0;; ++r) {
+    const int c = syrk_tiles(n, r);
+    if (x < c) {
+      const int all = (n - ROWS * r + 15) / 16, base = all / c, more = all % c;
+      return SyrkTile{ROWS * r, ROWS * r + 16 * (base * x + min(x, more)), base + (x < more ? 1 : 0)};
+    }
+    x -= c;
+  }
+}
+
+// One tile over steps [k0, k1) of 256 bytes a row, staged as the A = B C kernel
+// stages its own.
+template <class T, int NB>
+__device__ __forceinline__ void syrk_body(const typename T::X* __restrict__ X, int n, int i0, int j0, int k0, int k1,
+                                          u4* lds, typename T::P* __restrict__ out) {
+  typedef Waves<NB> W;
+  constexpr int RA = W::RA, NBW = W::NBW, PR = ROWS + 16 * NB;  // panel rows
+  constexpr int NC = PR * 16 / NT;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = w % W::M, wn = w / W::M;
+  const u4* src[NC];
+  u4 v[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int r = (t >> 4) + 16 * c;
+    const int row = min(r < ROWS ? i0 + r : j0 + r - ROWS, n - 1);  // rows past n repeat the last: never stored
+    src[c] = (const u4*)X + ((size_t)k0 * n + row) * 16 + (t & 15);
+  }
+  auto load = [&] {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      v[c] = *src[c];
+      src[c] += (size_t)n * 16;
+    }
+  };
+  typename T::acc acc[RA][NBW] = {};
+  if (k0 < k1) load();
+  for (int k = k0; k < k1; ++k) {
+    if (k > k0) __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int r = (t >> 4) + 16 * c;
+      lds[r * 16 + ((t & 15) ^ swz<16>(r))] = v[c];
+    }
+    if (k + 1 < k1) load();
+    __syncthreads();
+    step<T, 16>(acc, lds, lds + ROWS * 16, 16 * RA * wm, 16 * NBW * wn, lane);
+  }
+#pragma unroll
+  for (int a = 0; a < RA; ++a)
+#pragma unroll
+    for (int b = 0; b < NBW; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + 16 * (RA * wm + a) + T::row(lane, r), j = j0 + 16 * (NBW * wn + b) + (lane & 15);
+        if (i <= j && j < n) out[(size_t)i * n + j] = acc[a][b][r];
+      }
+}
+
+template <class T, int NB>
+__device__ __forceinline__ void syrk_pick(const SyrkTile& tl, const typename T::X* X, int n, int k0, int k1, u4* lds,
+                                          typename T::P* out) {
+  if constexpr (NB > 0) {
+    if (tl.nb != NB)
+      syrk_pick<T, NB - 1>(tl, X, n, k0, k1, lds, out);
+    else
+      syrk_body<T, NB>(X, n, tl.i0, tl.j0, k0, k1, lds, out);
+  }
+}
+
+// Workgroup (tile, slice): the tiles alone are far too few for 256 CUs, so the
+// contraction is cut into S slices (a multiple of 8) whose partial tiles a
+// second kernel sums in a fixed order.  Linear id 8 j + x runs on XCD x; it
+// takes slice x + 8 (j / tiles), so that every tile of a slice reads the
+// slice's panels through one L2.
+template <class T>
+__global__ __launch_bounds__(NT) void k_syrk(const typename T::X* __restrict__ X, int n, int steps, int S, int tiles,
+                                             typename T::P* __restrict__ part) {
+  __shared__ u4 lds[(ROWS + 160) * 16];
+  const int j = blockIdx.x / 8, s = blockIdx.x % 8 + 8 * (j / tiles);
+  const SyrkTile tl = syrk_tile(n, j % tiles);
+  const int k0 = (int)((long long)steps * s / S), k1 = (int)((long long)steps * (s + 1) / S);
+  syrk_pick<T, 10>(tl, X, n, k0, k1, lds, part + (size_t)s * n * n);
+}
+
+// K[i][j] = K[j][i] = alpha sum_s part[s][i][j], i <= j, by 32 x 32 tiles (both
+// writes along rows); the sums are in FP64 whatever the partials are.
+template <class P>
+__global__ __launch_bounds__(256) void k_syrk_reduce(const P* __restrict__ part, int S, int n, double alpha,
+                                                     double* __restrict__ K) {
+  __shared__ double tile[32][33];
+  if (blockIdx.y > blockIdx.x) return;
+  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  const size_t nn = (size_t)n * n;
+  for (int r = y; r < 32; r += 8) {
+    const int i = i0 + r, j = j0 + x;
+    double v = 0.0;
+    if (i <= j && j < n) {
+      const P* p = part + (size_t)i * n + j;
+      for (int s = 0; s < S; ++s) v += (double)p[s * nn];
+      v *= alpha;
+      K[(size_t)i * n + j] = v;
+    }
+    tile[r][x] = v;
+  }
+  __syncthreads();
+  for (int r = y; r < 32; r += 8) {
+    const int j = j0 + r, i = i0 + x;
+    if (i < j && j < n) K[(size_t)j * n + i] = tile[x][r];
+  }
+}
+
+template <class T>
+void k_from_tiles(const double* Bt, size_t npt, int rank, int n, const double* C, int o, double* K, double* gamma,
+                  ExchangeWork& w, hipStream_t st) {
+  typedef typename T::X X;
+  typedef typename T::P P;
+  const int nt = tiles_of(n);
+  int nb = 0, gy = 0;
+  column_tiles(o, nb, gy);
+  const int an = 16 * nb;
+  const long long L = (long long)rank * o, steps = (L + T::XK - 1) / T::XK;
+  if (steps > INT32_MAX) throw HfgError{HFG_UNSUPPORTED, "DF exchange: contraction index out of range"};
+  int tiles = 0;
+  for (int r = 0; ROWS * r < n; ++r) tiles += syrk_tiles(n, r);
+  // slices: about six rounds of the chip's 512 workgroups (two a CU), at least
+  // four steps each, a multiple of 8
+  long long S = (3072 + tiles - 1) / tiles;
+  S = std::min(S, std::max<long long>(1, steps / 4));
+  S = (S + 7) / 8 * 8;
+  w.c.grow((size_t)gy * nt * an * T::CH * 16);
+  w.x.grow((size_t)steps * n * 256);
+  w.part.grow((size_t)S * n * n * sizeof(P));
+  double* part = nullptr;
+  if (gamma) {
+    w.sums.grow((size_t)rank * nt * 2 * gy * 8);
+    part = w.sums.template as<double>();
+  }
+  u4* cp = w.c.template as<u4>();
+  X* x = w.x.template as<X>();
+  hipLaunchKernelGGL(k_pack_c<T>, dim3((unsigned)((gy * nt * an * 16 + 255) / 256)), dim3(256), 0, st, C, n, o, nt, an,
+                     gy, cp);
   HIP_CHECK(hipGetLastError());
-  const unsigned gx = (unsigned)((n + SM - 1) / SM), gy = (unsigned)(oc / SN);
-  const long long total = (long long)gx * gy * rank;
-  if (total > INT32_MAX) throw HfgError{HFG_UNSUPPORTED, "packed A = B C: too many tiles for one launch"};
-  hipLaunchKernelGGL(k_bc_packed_bf16x3, dim3((unsigned)total), dim3(512), 0, st, Bp, np, n, Th, Tl, nk, o, Ah, Al,
-                     ldt, (int)gx, (int)gy, total, BC_XCD_MAP | BC_TOURNAMENT);
+  if (const int w = (int)(steps * T::XK - L)) {
+    hipLaunchKernelGGL(k_zero_tail<X>, dim3((unsigned)((w * n + 255) / 256)), dim3(256), 0, st, x, n, L, w);
+    HIP_CHECK(hipGetLastError());
+  }
+  launch_bc<T, 10>(nb, Bt, npt, nt, rank, n, cp, C, o, x, part, gy, st);
+  if (gamma) {
+    hipLaunchKernelGGL(k_part_reduce, dim3((unsigned)((rank + 255) / 256)), dim3(256), 0, st, part, nt * 2 * gy, rank,
+                       2.0, gamma);
+    HIP_CHECK(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_syrk<T>, dim3((unsigned)(tiles * S)), dim3(NT), 0, st, x, n, (int)steps, (int)S, tiles,
+                     w.part.template as<P>());
+  HIP_CHECK(hipGetLastError());
+  const unsigned g = (unsigned)((n + 31) / 32);
+  hipLaunchKernelGGL(k_syrk_reduce<P>, dim3(g, g), dim3(256), 0, st, w.part.template as<P>(), (int)S, n, 2.0, K);
   HIP_CHECK(hipGetLastError());
 }
 
-// Contraction slices for an n x n output and contraction length L: enough
-// workgroups (about 2048) for the chip, at least 64 of L each, at most 64.
-size_t syrk_f64_slices(int n, long long L) {
-  const long long nt = (n + ST - 1) / ST, upper = nt * (nt + 1) / 2;
-  long long s = std::max<long long>(1, (2048 + upper - 1) / upper);
-  s = std::min<long long>(s, std::max<long long>(1, L / (4 * KB)));  // at least 64 of L per slice
-  return (size_t)std::min<long long>(s, 64);
-}
+}  // namespace
 
-// K = alpha X X^T, X row-major n x L (leading dimension ldx), K row-major
-// n x n (both triangles), on stream st; scratch grows to the partial tiles
-// (slices x n x n doubles) and the tile list.
-void syrk_f64(const double* X, int n, long long L, long long ldx, double alpha, double* K, DevBuf& scratch,
-              hipStream_t st) {
-  const int nt = (n + ST - 1) / ST;
-  const int upper = nt * (nt + 1) / 2;
-  const int S = (int)syrk_f64_slices(n, L);
-  const size_t need = (size_t)S * n * n * sizeof(double) + (size_t)upper * sizeof(int2);
-  if (scratch.bytes < need) scratch.alloc(need);
-  double* part = scratch.as<double>();
-  int2* tiles = (int2*)(scratch.as<char>() + (size_t)S * n * n * sizeof(double));
-  std::vector<int2> h;
-  h.reserve(upper);
-  for (int a = 0; a < nt; ++a)
-    for (int b = a; b < nt; ++b) h.push_back(make_int2(a, b));
-  HIP_CHECK(hipMemcpyAsync(tiles, h.data(), h.size() * sizeof(int2), hipMemcpyHostToDevice, st));
-  const long long kslice = ((L + S - 1) / S + KB - 1) / KB * KB;
-  hipLaunchKernelGGL(k_syrk_f64, dim3((unsigned)(upper * S)), dim3(SYRK_NT), 0, st, X, n, L, ldx, tiles, upper,
-                     kslice, part);
-  HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_syrk_reduce, dim3(2048), dim3(256), 0, st, part, S, n, alpha, K);
-  HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipStreamSynchronize(st));  // the tile list is a host vector
+void df_exchange(const double* Bt, size_t npt, int rank, int n, const double* C, int o, int precision, double* K,
+                 double* gamma, ExchangeWork& w, hipStream_t st) {
+  if (precision == 0)
+    k_from_tiles<F64>(Bt, npt, rank, n, C, o, K, gamma, w, st);
+  else if (precision == 1)
+    k_from_tiles<F32>(Bt, npt, rank, n, C, o, K, nullptr, w, st);
+  else
+    k_from_tiles<BF16x3>(Bt, npt, rank, n, C, o, K, nullptr, w, st);
 }
 
 }  // namespace hfg
