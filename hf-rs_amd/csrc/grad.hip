@@ -13,20 +13,15 @@
 // classes of gen/eri_grad.inc); one kernel then contracts every block with G
 // and adds the quartet's forces to per-workgroup LDS sums of the atoms' forces.
 //
-// One-electron part on the host (the size of a Fock-matrix set-up): the
-// overlap, kinetic and nuclear-attraction derivatives of each basis function
-// (src/gradient.rs:411-447), the operator derivative of the attraction at each
-// nucleus (:451-490), and the nuclear repulsion (:220-243).
+// One-electron terms on the device (onee_dev.hip); the nuclear repulsion
+// (src/gradient.rs:220-243) on the host.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <array>
-#include <chrono>
-#include <cstdio>
-#include <cstdlib>
 #include <cmath>
 #include <cstring>
-#include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/hfg.h"
@@ -121,105 +116,139 @@ constexpr CartTab make_cart() {
   }
   return t;
 }
-__constant__ CartTab g_cart = make_cart();
+const CartTab g_cart = make_cart();
 
-// One derivative block of a quartet: storage position p (0..3: first pair's
-// first and second shell, second pair's first and second shell) holds
-// original shell sh[p] (0..3 = A, B, C, D of the quartet) with angular
-// momentum L[p]; position mod holds the raised (raised = 1) or lowered shell
-// whose centre is differentiated.
-struct GBlock {
-  long long off;
-  signed char sh[4], L[4];
-  signed char mod, raised, pad[2];
-};
-// A quartet: its shells' AO offsets, angular momenta and atoms; its blocks;
-// w = 1/2 x degeneracy.
-struct GQuartet {
-  int ao[4];
-  int atom[4];
-  signed char L[4];
-  int nblk;
-  GBlock blk[6];
-  double w;
+// A shell pair as the gradient's kernels read it: AO offsets and atoms of its
+// two shells (kernel orientation), and its four derivative pairs' entries in
+// the pair table (raised and lowered first shell, raised and lowered second;
+// -1: none).
+struct GPair {
+  int ao[2], atom[2], d[4];
 };
 
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// The quartets of a pair of pair classes (la lb|lc ld) all have the same
+// derivative blocks: at most six (raised and lowered A, B and C).
+constexpr int MAX_BLK = 6;
+struct GBlocks {
+  int n;
+  int ket[MAX_BLK];    // the derivative pair is the ket's (of C), else the bra's
+  int slot[MAX_BLK];   // which of the pair's derivative pairs
+  int first[MAX_BLK];  // the block stores the derivative pair first
+  int size[MAX_BLK];
+  long long base[MAX_BLK];  // of the block's batch in the block buffer
+};
+
+// Quartet t of a class: rows are the bra class's pairs, each with the prefix of
+// the ket class's pairs (both sorted by Schwarz bound) that passes the test;
+// pre[i] .. pre[i + 1] - 1 are row i's.  Writes the quartet's pairs and its block
+// tasks (block by block, nq each).  One thread a quartet: on the host, listing
+// the quartets of C8H18/6-31G and copying the lists took 130 of 162 ms; the
+// whole gradient is now 19.4 ms.
+__global__ __launch_bounds__(256) void k_grad_tasks(const int* __restrict__ bra, const int* __restrict__ ket,
+                                                    const long long* __restrict__ pre, int rows, long long t0, int nq,
+                                                    const GPair* __restrict__ pairs, GBlocks g,
+                                                    int2* __restrict__ quartets, BlockTask* __restrict__ tasks) {
+  const int q = blockIdx.x * 256 + threadIdx.x;
+  if (q >= nq) return;
+  const long long t = t0 + q;
+  int lo = 0, hi = rows - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (pre[mid] <= t)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  const int ij = bra[lo], kl = ket[t - pre[lo]];
+  quartets[q] = int2{ij, kl};
+  for (int b = 0; b < g.n; ++b) {
+    const int dp = pairs[g.ket[b] ? kl : ij].d[g.slot[b]], other = g.ket[b] ? ij : kl;
+    tasks[(size_t)b * nq + q] =
+        BlockTask{g.first[b] ? dp : other, g.first[b] ? other : dp, g.base[b] + (long long)q * g.size[b]};
+  }
 }
 
-// Contraction of every quartet's derivative blocks with G: one wave per
-// quartet (waves stride over the list), forces summed per atom in LDS, added
-// to grad (natom x 3) at the end.
-__global__ __launch_bounds__(256) void k_grad_contract(const GQuartet* __restrict__ qs, int nq,
+// One term of a quartet's force: element e of block b times coef contributes,
+// with G of the quartet's own element o, to one derivative (x, y or z of A, B
+// or C; the entries are grouped by it).
+struct GEntry {
+  unsigned short o, e;
+  short b, coef;
+};
+struct GContract {
+  int dim[4];       // components of A, B, C, D
+  int end[9];       // entries up to derivative s (A x, y, z, B x, ...)
+  GBlocks blocks;
+};
+
+// Forces of every quartet: G = P_mn P_ls - 1/4 (P_ml P_ns + P_ms P_nl) with the
+// component factors, each of its elements once into LDS, then the entries, the
+// nine sums and d/dD = -(d/dA + d/dB + d/dC).  GL lanes a quartet, chosen by
+// the class's entries (9 for (ss|ss), 1,197 for (pp|pp)): a wave per quartet
+// had 3 of 64 lanes at work on an (ss|ss) block and formed G again for every
+// entry.  Atoms' forces are summed in LDS per workgroup, then added to grad
+// (natom x 3).  w = 1/2 x the quartet's degeneracy.
+template <int GL>
+__global__ __launch_bounds__(256) void k_grad_contract(const int2* __restrict__ quartets, int nq,
+                                                       const GPair* __restrict__ pairs, GContract c,
+                                                       const GEntry* __restrict__ entries,
                                                        const double* __restrict__ blk, const double* __restrict__ P,
                                                        const double* __restrict__ scale, int n, int natom,
                                                        double* __restrict__ grad) {
-  extern __shared__ double acc[];  // natom x 3
+  extern __shared__ double lds[];
+  const int nt = c.dim[0] * c.dim[1] * c.dim[2] * c.dim[3];
+  double* acc = lds;                                           // natom x 3
+  double* G = lds + 3 * natom + (size_t)(threadIdx.x / GL) * nt;  // this group's quartet
   for (int i = threadIdx.x; i < 3 * natom; i += blockDim.x) acc[i] = 0.0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int waves = gridDim.x * (blockDim.x >> 6);
-  for (int q = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); q < nq; q += waves) {
-    const GQuartet& Q = qs[q];
-    double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};  // d/dA, d/dB, d/dC (x, y, z)
-    for (int b = 0; b < Q.nblk; ++b) {
-      const GBlock B = Q.blk[b];
-      const int n0 = ncart(B.L[0]), n1 = ncart(B.L[1]), n2 = ncart(B.L[2]), n3 = ncart(B.L[3]);
-      const int ne = n0 * n1 * n2 * n3;
-      const int X = B.sh[B.mod];                 // differentiated shell (0, 1 or 2)
-      const int Lo = Q.L[X];                     // its own angular momentum
-      for (int e = lane; e < ne; e += 64) {
-        int c[4];
-        c[3] = e % n3;
-        c[2] = (e / n3) % n2;
-        c[1] = (e / (n3 * n2)) % n1;
-        c[0] = e / (n3 * n2 * n1);
-        const double v = blk[B.off + e];
-        int o[4];
-        for (int p = 0; p < 4; ++p) o[B.sh[p]] = c[p];
-        const signed char* ex = g_cart.e[B.L[B.mod]][c[B.mod]];
-        for (int t = 0; t < 3; ++t) {
-          int ee[3] = {ex[0], ex[1], ex[2]};
-          double coef;
-          if (B.raised) {
-            if (ee[t] == 0) continue;
-            --ee[t];
-            coef = 1.0;
-          } else {
-            coef = -(double)(ee[t] + 1);
-            ++ee[t];
-          }
-          o[X] = g_cart.idx[Lo][ee[0]][ee[1]];
-          const int mu = Q.ao[0] + o[0], nu = Q.ao[1] + o[1], la = Q.ao[2] + o[2], si = Q.ao[3] + o[3];
-          const double G = P[(size_t)mu * n + nu] * P[(size_t)la * n + si] -
-                           0.25 * (P[(size_t)mu * n + la] * P[(size_t)nu * n + si] +
-                                   P[(size_t)mu * n + si] * P[(size_t)nu * n + la]);
-          const double c = coef * v * G * scale[mu] * scale[nu] * scale[la] * scale[si];
-          if (X == 0)
-            gA[t] += c;
-          else if (X == 1)
-            gB[t] += c;
-          else
-            gC[t] += c;
-        }
+  const int lane = threadIdx.x % GL, per = 256 / GL;
+  const int rounds = (nq + per * gridDim.x - 1) / (per * gridDim.x);
+  for (int r = 0; r < rounds; ++r) {
+    const int q = (r * gridDim.x + blockIdx.x) * per + threadIdx.x / GL;
+    const bool on = q < nq;
+    const int2 ids = quartets[on ? q : 0];
+    const GPair A = pairs[ids.x], C = pairs[ids.y];
+    __syncthreads();  // the last round's G is read, and acc is clear
+    if (on)
+      for (int o = lane; o < nt; o += GL) {
+        int x = o;
+        const int d = x % c.dim[3];
+        x /= c.dim[3];
+        const int cc = x % c.dim[2];
+        x /= c.dim[2];
+        const int b = x % c.dim[1], a = x / c.dim[1];
+        const size_t mu = A.ao[0] + a, nu = A.ao[1] + b, la = C.ao[0] + cc, si = C.ao[1] + d;
+        G[o] = (P[mu * n + nu] * P[la * n + si] -
+                0.25 * (P[mu * n + la] * P[nu * n + si] + P[mu * n + si] * P[nu * n + la])) *
+               scale[mu] * scale[nu] * scale[la] * scale[si];
       }
-    }
+    __syncthreads();
     double s[9];
-    for (int t = 0; t < 3; ++t) {
-      s[t] = wave_sum(gA[t]) * Q.w;
-      s[3 + t] = wave_sum(gB[t]) * Q.w;
-      s[6 + t] = wave_sum(gC[t]) * Q.w;
+    int k = lane;
+#pragma unroll
+    for (int x = 0; x < 9; ++x) {
+      double v = 0.0;
+      if (on)
+        for (; k < c.end[x]; k += GL) {
+          const GEntry e = entries[k];
+          v += e.coef * blk[c.blocks.base[e.b] + (long long)q * c.blocks.size[e.b] + e.e] * G[e.o];
+        }
+#pragma unroll
+      for (int o = GL / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, GL);
+      s[x] = v;
     }
-    if (lane == 0)
+    if (on && lane == 0) {
+      double w = 0.5;
+      if (A.ao[0] != A.ao[1]) w *= 2.0;
+      if (C.ao[0] != C.ao[1]) w *= 2.0;
+      if (ids.x != ids.y) w *= 2.0;
+#pragma unroll
       for (int t = 0; t < 3; ++t) {
-        atomicAdd(&acc[3 * Q.atom[0] + t], s[t]);
-        atomicAdd(&acc[3 * Q.atom[1] + t], s[3 + t]);
-        atomicAdd(&acc[3 * Q.atom[2] + t], s[6 + t]);
-        atomicAdd(&acc[3 * Q.atom[3] + t], -(s[t] + s[3 + t] + s[6 + t]));
+        atomicAdd(&acc[3 * A.atom[0] + t], w * s[t]);
+        atomicAdd(&acc[3 * A.atom[1] + t], w * s[3 + t]);
+        atomicAdd(&acc[3 * C.atom[0] + t], w * s[6 + t]);
+        atomicAdd(&acc[3 * C.atom[1] + t], -w * (s[t] + s[3 + t] + s[6 + t]));
       }
+    }
   }
   __syncthreads();
   for (int i = threadIdx.x; i < 3 * natom; i += blockDim.x)
@@ -238,12 +267,80 @@ Shell lowered(const Shell& s) {
   return r;
 }
 
-// The derivative pairs of one shell pair (kernel orientation A, B): raised
-// and lowered A, raised and lowered B, each stored with the higher L first.
-struct DPair {
-  int idx[4] = {-1, -1, -1, -1};   // pair-table entry: RA, LA, RB, LB
-  bool swap[4] = {false, false, false, false};  // stored as (B', A) / (B, A')
+// The blocks and force terms of class (L0 L1|L2 L3).  A block's derivative pair
+// is stored with the higher L first, and the pair of higher rank first in the
+// block.
+struct GClass {
+  GBlocks blocks = {};
+  int key[MAX_BLK][4];  // the blocks' own classes
+  GContract c = {};
+  std::vector<GEntry> entries;
 };
+GClass gradient_class(const int (&L)[4]) {
+  GClass k;
+  std::vector<GEntry> by[9];
+  auto add = [&](int X, bool up) {  // raised or lowered shell X (0, 1 or 2)
+    const int l = L[X] + (up ? 1 : -1), side = X / 2, Y = X ^ 1;  // Y: X's partner
+    if (l < 0) return;
+    const int b = k.blocks.n++;
+    // X before Y unless its L is now the lower one; first shells stay first at equal L
+    const bool x_first = X % 2 ? l > L[Y] : l >= L[Y];
+    const int d0 = x_first ? X : Y, d1 = x_first ? Y : X, o0 = side ? 0 : 2, o1 = o0 + 1;
+    auto len = [&](int s) { return s == X ? l : L[s]; };
+    const bool first = pair_rank(len(d0), len(d1)) >= pair_rank(L[o0], L[o1]);
+    const int sh[4] = {first ? d0 : o0, first ? d1 : o1, first ? o0 : d0, first ? o1 : d1};
+    int dim[4], size = 1;
+    for (int p = 0; p < 4; ++p) {
+      k.key[b][p] = len(sh[p]);
+      dim[p] = ncart(len(sh[p]));
+      size *= dim[p];
+    }
+    k.blocks.ket[b] = side;
+    k.blocks.slot[b] = 2 * (X % 2) + (up ? 0 : 1);
+    k.blocks.first[b] = first;
+    k.blocks.size[b] = size;
+    for (int e = 0; e < size; ++e) {
+      int o[4], r = e;
+      for (int p = 3; p >= 0; --p) {
+        o[sh[p]] = r % dim[p];
+        r /= dim[p];
+      }
+      const signed char* ex = g_cart.e[l][o[X]];
+      for (int t = 0; t < 3; ++t) {
+        int ee[3] = {ex[0], ex[1], ex[2]};
+        if (up && ee[t] == 0) continue;
+        const int coef = up ? 1 : -(ee[t] + 1);
+        ee[t] += up ? -1 : 1;
+        int own[4] = {o[0], o[1], o[2], o[3]};
+        own[X] = g_cart.idx[L[X]][ee[0]][ee[1]];
+        const int at = ((own[0] * ncart(L[1]) + own[1]) * ncart(L[2]) + own[2]) * ncart(L[3]) + own[3];
+        by[3 * X + t].push_back(GEntry{(unsigned short)at, (unsigned short)e, (short)b, (short)coef});
+      }
+    }
+  };
+  for (int X = 0; X < 3; ++X)
+    for (bool up : {true, false}) add(X, up);
+  for (int p = 0; p < 4; ++p) k.c.dim[p] = ncart(L[p]);
+  for (int x = 0; x < 9; ++x) {
+    k.entries.insert(k.entries.end(), by[x].begin(), by[x].end());
+    k.c.end[x] = (int)k.entries.size();
+  }
+  return k;
+}
+
+template <int GL>
+void launch_contract(const GContract& c, const int2* quartets, int nq, const GPair* pairs, const GEntry* entries,
+                     const double* blk, const double* P, const double* scale, int n, int natom, double* grad,
+                     hipStream_t st) {
+  const size_t lds = (3 * (size_t)natom + (size_t)(256 / GL) * c.dim[0] * c.dim[1] * c.dim[2] * c.dim[3]) * 8;
+  if (lds > 65536)
+    HIP_CHECK(hipFuncSetAttribute((const void*)k_grad_contract<GL>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)lds));
+  const int blocks = std::min(2048, (nq + 256 / GL - 1) / (256 / GL));
+  hipLaunchKernelGGL(k_grad_contract<GL>, dim3(blocks), dim3(256), lds, st, quartets, nq, pairs, c, entries, blk, P,
+                     scale, n, natom, grad);
+  HIP_CHECK(hipGetLastError());
+}
 
 }  // namespace
 
@@ -272,45 +369,56 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
   const std::vector<Shell>& sh = e.shells;
   const std::vector<double>& sc = e.ao_scale;
   // ---- two-electron part on the device
+  // pair table: the engine's pairs, then the derivative pairs (raised and
+  // lowered first shell, raised and lowered second), each with the higher L
+  // first; filled in parallel at offsets fixed in advance
   const size_t npair = e.pairs.size();
-  // pair table: the engine's pairs, then the derivative pairs
+  std::vector<GPair> gp(npair);
+  std::vector<size_t> off(4 * npair + 1, e.pp.size());
+  std::vector<int> slots;  // pair * 4 + slot of the derivative pairs, in table order
+  for (size_t i = 0; i < npair; ++i) {
+    const PairInfo& p = e.pairs[i];
+    GPair& g_ = gp[i];
+    g_ = GPair{{p.ao_a, p.ao_b}, {sh[p.sh_a].atom, sh[p.sh_b].atom}, {-1, -1, -1, -1}};
+    const size_t prims = (size_t)sh[p.sh_a].K * sh[p.sh_b].K;
+    for (int s = 0; s < 4; ++s) {
+      const bool have = s == 0 || s == 2 || (s == 1 ? p.la : p.lb) > 0;
+      if (have) {
+        g_.d[s] = (int)(npair + slots.size());
+        slots.push_back((int)(4 * i + s));
+      }
+      off[4 * i + s + 1] = off[4 * i + s] + (have ? prims : 0);
+    }
+  }
   PrimPairHost pp = e.pp;
-  std::vector<PairDev> pd(npair);
-  std::vector<std::array<int, 2>> pl(npair);  // (L first, L second) per table entry
+  std::vector<double>* grow[9] = {&pp.p, &pp.Px, &pp.Py, &pp.Pz, &pp.PAx, &pp.PAy, &pp.PAz, &pp.K, &pp.H};
+  for (auto* c : grow) c->resize(off.back());
+  std::vector<PairDev> pd(npair + slots.size());
   for (size_t i = 0; i < npair; ++i) {
     const PairInfo& p = e.pairs[i];
     std::memset(&pd[i], 0, sizeof(PairDev));
     pd[i].p0 = p.p0;
     pd[i].p1 = p.p1;
     for (int k = 0; k < 3; ++k) pd[i].AB[k] = p.AB[k];
-    pl[i] = {p.la, p.lb};
   }
-  auto add_pair = [&](const Shell& X, const Shell& Y) {
-    PairDev d;
-    std::memset(&d, 0, sizeof d);
-    d.p0 = (int)pp.size();
-    append_pair(X, Y, pp);
-    d.p1 = (int)pp.size();
-    for (int k = 0; k < 3; ++k) d.AB[k] = X.c[k] - Y.c[k];
-    pd.push_back(d);
-    pl.push_back({X.L, Y.L});
-    return (int)pd.size() - 1;
-  };
-  std::vector<DPair> dp(npair);
-  for (size_t i = 0; i < npair; ++i) {
-    const PairInfo& p = e.pairs[i];
+#pragma omp parallel for schedule(dynamic, 64)
+  for (long x = 0; x < (long)slots.size(); ++x) {
+    const PairInfo& p = e.pairs[slots[x] / 4];
+    const int s = slots[x] % 4;
     const Shell &A = sh[p.sh_a], &B = sh[p.sh_b];
-    DPair& d = dp[i];
-    d.idx[0] = add_pair(raised(A), B);  // L_A + 1 > L_B
-    if (A.L > 0) {
-      const Shell la = lowered(A);
-      d.swap[1] = la.L < B.L;
-      d.idx[1] = d.swap[1] ? add_pair(B, la) : add_pair(la, B);
-    }
-    const Shell rb = raised(B);
-    d.swap[2] = rb.L > A.L;
-    d.idx[2] = d.swap[2] ? add_pair(rb, A) : add_pair(A, rb);
-    if (B.L > 0) d.idx[3] = add_pair(A, lowered(B));  // L_A >= L_B - 1
+    const Shell D = s == 0 ? raised(A) : s == 1 ? lowered(A) : s == 2 ? raised(B) : lowered(B);
+    const bool d_first = s < 2 ? D.L >= B.L : D.L > A.L;
+    const Shell &X = s < 2 ? (d_first ? D : B) : (d_first ? D : A), &Y = s < 2 ? (d_first ? B : D) : (d_first ? A : D);
+    PrimPairHost one;
+    append_pair(X, Y, one);
+    const size_t at = off[slots[x]];
+    const std::vector<double>* from[9] = {&one.p, &one.Px, &one.Py, &one.Pz, &one.PAx, &one.PAy, &one.PAz, &one.K, &one.H};
+    for (int c = 0; c < 9; ++c) std::copy(from[c]->begin(), from[c]->end(), grow[c]->begin() + at);
+    PairDev& d = pd[npair + x];
+    std::memset(&d, 0, sizeof d);
+    d.p0 = (int)at;
+    d.p1 = (int)(at + one.size());
+    for (int k = 0; k < 3; ++k) d.AB[k] = X.c[k] - Y.c[k];
   }
   const size_t npp = pp.size();
   DevBuf d_pp, d_pd, d_scale, d_grad;
@@ -329,194 +437,109 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
   const double* b = d_pp.as<double>();
   const PrimPairs view{b, b + npp, b + 2 * npp, b + 3 * npp, b + 4 * npp, b + 5 * npp, b + 6 * npp, b + 7 * npp,
                        b + 8 * npp};
-  // The quartets of pair rows ij (kl <= ij, passing the Schwarz test) and
-  // their derivative blocks.  A counting pass (parallel over rows) gives each
-  // row's quartet, block and block-double counts; consecutive rows form
-  // batches of at most `budget` block doubles; a second parallel pass fills
-  // each row's segment of the batch, and the block tasks are bucketed by
-  // class (row order kept within a class) for one launch per class.
+  // Quartets by pair of pair classes: both classes' pairs sorted by Schwarz
+  // bound, so that the ket pairs of a row that pass the test are a prefix (and
+  // of one class with itself the rows' earlier pairs).  The lists are written on
+  // the device, in batches of at most BUDGET block doubles.
   const size_t lds = (size_t)3 * na * sizeof(double);
   if (lds > 60000) throw HfgError{HFG_UNSUPPORTED, "gradient: too many atoms for the per-workgroup force sums"};
-  const bool trace = std::getenv("HFG_TRACE") != nullptr;
-  auto now = [] { return std::chrono::steady_clock::now(); };
-  auto secs = [](std::chrono::steady_clock::time_point t0, std::chrono::steady_clock::time_point t1) {
-    return std::chrono::duration<double>(t1 - t0).count();
-  };
-  const auto t_start = now();
-  double t_count = 0, t_fill = 0, t_gpu = 0;
-  auto cls_key = [](int l0, int l1, int l2, int l3) { return ((l0 * 5 + l1) * 5 + l2) * 5 + l3; };
-  constexpr int NKEY = 625;
-  // One block of a quartet: derivative pair dpi against pair other.  With Q
-  // null only the block's size is returned.
-  auto add_block = [&](GQuartet* Q, long long& off, BlockTask* t_out, int* k_out, int dpi, bool dswap, int other,
-                       const int sh_d[2], const int sh_o[2], bool raised_) -> long long {
-    const std::array<int, 2> ld = pl[dpi], lo = pl[other];
-    const long long size = (long long)ncart(ld[0]) * ncart(ld[1]) * ncart(lo[0]) * ncart(lo[1]);
-    if (!Q) return size;
-    // storage: the pair of higher rank first
-    const bool dfirst = pair_rank(ld[0], ld[1]) >= pair_rank(lo[0], lo[1]);
-    GBlock& B = Q->blk[Q->nblk++];
-    B.off = off;
-    B.raised = raised_ ? 1 : 0;
-    const int dpos0 = dfirst ? 0 : 2, opos0 = dfirst ? 2 : 0;
-    // derivative pair storage order: (mod, partner) unless swapped
-    B.sh[dpos0] = (signed char)(dswap ? sh_d[1] : sh_d[0]);
-    B.sh[dpos0 + 1] = (signed char)(dswap ? sh_d[0] : sh_d[1]);
-    B.L[dpos0] = (signed char)ld[0];
-    B.L[dpos0 + 1] = (signed char)ld[1];
-    B.mod = (signed char)(dswap ? dpos0 + 1 : dpos0);
-    B.sh[opos0] = (signed char)sh_o[0];
-    B.sh[opos0 + 1] = (signed char)sh_o[1];
-    B.L[opos0] = (signed char)lo[0];
-    B.L[opos0 + 1] = (signed char)lo[1];
-    if (dfirst) {
-      *k_out = cls_key(ld[0], ld[1], lo[0], lo[1]);
-      *t_out = BlockTask{dpi, other, off};
-    } else {
-      *k_out = cls_key(lo[0], lo[1], ld[0], ld[1]);
-      *t_out = BlockTask{other, dpi, off};
-    }
-    off += size;
-    return size;
-  };
-  // Quartet (ij, kl): its blocks (d/dA raised and lowered, d/dB raised and
-  // lowered, d/dC raised and lowered); returns the block count and adds the
-  // block doubles to off.  Count-only with Q null.
-  auto make_quartet = [&](size_t ij, size_t kl, GQuartet* Q, BlockTask* t_out, int* k_out, long long& off) {
-    const PairInfo& pb = e.pairs[ij];
-    const PairInfo& pk = e.pairs[kl];
-    if (Q) {
-      std::memset(Q, 0, sizeof *Q);
-      const int shells4[4] = {pb.sh_a, pb.sh_b, pk.sh_a, pk.sh_b};
-      for (int k = 0; k < 4; ++k) {
-        const Shell& s = sh[shells4[k]];
-        Q->ao[k] = s.ao;
-        Q->atom[k] = s.atom;
-        Q->L[k] = (signed char)s.L;
-      }
-      double deg = 1.0;
-      if (pb.sh_a != pb.sh_b) deg *= 2.0;
-      if (pk.sh_a != pk.sh_b) deg *= 2.0;
-      if (ij != kl) deg *= 2.0;
-      Q->w = 0.5 * deg;
-    }
-    const int AB[2] = {0, 1}, BA[2] = {1, 0}, CD[2] = {2, 3};
-    const DPair& db = dp[ij];
-    const DPair& dk = dp[kl];
-    int nb = 0;
-    long long count_off = 0;
-    long long& o = Q ? off : count_off;
-    auto add = [&](int dpi, bool dswap, int other, const int* sd, const int* so, bool r) {
-      const long long sz = add_block(Q, o, t_out + nb, k_out + nb, dpi, dswap, other, sd, so, r);
-      if (!Q) o += sz;
-      ++nb;
-    };
-    add(db.idx[0], false, (int)kl, AB, CD, true);
-    if (db.idx[1] >= 0) add(db.idx[1], db.swap[1], (int)kl, AB, CD, false);
-    add(db.idx[2], !db.swap[2], (int)kl, BA, CD, true);
-    if (db.idx[3] >= 0) add(db.idx[3], true, (int)kl, BA, CD, false);
-    add(dk.idx[0], false, (int)ij, CD, AB, true);
-    if (dk.idx[1] >= 0) add(dk.idx[1], dk.swap[1], (int)ij, CD, AB, false);
-    if (!Q) off += count_off;
-    return nb;
-  };
-  // counting pass
-  std::vector<long long> row_q(npair), row_b(npair), row_d(npair);
-  {
-    const auto t0 = now();
-#pragma omp parallel for schedule(dynamic, 16)
-    for (long long ij = 0; ij < (long long)npair; ++ij) {
-      long long q = 0, nb = 0, d = 0;
-      for (size_t kl = 0; kl <= (size_t)ij; ++kl) {
-        if (!(e.Q[ij] * e.Q[kl] > e.screen)) continue;
-        ++q;
-        nb += make_quartet((size_t)ij, kl, nullptr, nullptr, nullptr, d);
-      }
-      row_q[ij] = q;
-      row_b[ij] = nb;
-      row_d[ij] = d;
-    }
-    t_count = secs(t0, now());
+  std::array<std::vector<int>, 6> cls;  // pairs by class, largest bound first
+  for (size_t i = 0; i < npair; ++i) cls[pair_class(e.pairs[i].la, e.pairs[i].lb)].push_back((int)i);
+  std::vector<int> order;
+  std::array<size_t, 6> at = {};
+  for (int c = 0; c < 6; ++c) {
+    std::stable_sort(cls[c].begin(), cls[c].end(), [&](int x, int y) { return e.Q[x] > e.Q[y]; });
+    at[c] = order.size();
+    order.insert(order.end(), cls[c].begin(), cls[c].end());
   }
-  const long long budget = 1ll << 26;  // block doubles per batch (512 MB)
-  DevBuf d_tasks, d_blk, d_q;
-  size_t cap_t = 0, cap_b = 0, cap_q = 0;
-  std::vector<GQuartet> quartets;
-  std::vector<BlockTask> rtask, tasks;
-  std::vector<int> rkey;
-  size_t r0 = 0;
-  int batches = 0;
-  while (r0 < npair) {
-    // rows [r0, r1): at least one row, then as many as fit the budget
-    size_t r1 = r0 + 1;
-    long long dsum = row_d[r0];
-    while (r1 < npair && dsum + row_d[r1] <= budget) dsum += row_d[r1++];
-    std::vector<long long> qo(r1 - r0 + 1, 0), bo(r1 - r0 + 1, 0), dof(r1 - r0 + 1, 0);
-    for (size_t r = r0; r < r1; ++r) {
-      qo[r - r0 + 1] = qo[r - r0] + row_q[r];
-      bo[r - r0 + 1] = bo[r - r0] + row_b[r];
-      dof[r - r0 + 1] = dof[r - r0] + row_d[r];
-    }
-    const size_t nq = (size_t)qo.back(), nbk = (size_t)bo.back();
-    const long long ndbl = dof.back();
-    r0 = r1;
-    if (nq == 0) continue;
-    const auto t0 = now();
-    quartets.resize(nq);
-    rtask.resize(nbk);
-    rkey.resize(nbk);
-    const size_t rbase = r1 - (qo.size() - 1);
-#pragma omp parallel for schedule(dynamic, 16)
-    for (long long r = 0; r < (long long)(qo.size() - 1); ++r) {
-      const size_t ij = rbase + (size_t)r;
-      long long qi = qo[r], bi = bo[r], off = dof[r];
-      for (size_t kl = 0; kl <= ij; ++kl) {
-        if (!(e.Q[ij] * e.Q[kl] > e.screen)) continue;
-        bi += make_quartet(ij, kl, &quartets[qi], &rtask[bi], &rkey[bi], off);
-        ++qi;
+  struct Job {
+    int cb, ck;
+    size_t pre;  // of its rows' prefix sums
+    long long total;
+    GClass g;
+    size_t entries;
+  };
+  std::vector<Job> jobs;
+  std::vector<long long> pre;
+  std::vector<GEntry> entries;
+  for (int cb = 0; cb < 6; ++cb)
+    for (int ck = 0; ck <= cb; ++ck) {
+      if (cls[cb].empty() || cls[ck].empty()) continue;
+      Job j{cb, ck, pre.size(), 0, {}, entries.size()};
+      size_t hi = cls[ck].size();  // falls with the row's bound
+      for (size_t i = 0; i < cls[cb].size(); ++i) {
+        pre.push_back(j.total);
+        while (hi > 0 && !(e.Q[cls[cb][i]] * e.Q[cls[ck][hi - 1]] > e.screen)) --hi;
+        j.total += (long long)(cb == ck ? std::min(hi, i + 1) : hi);
       }
+      pre.push_back(j.total);
+      if (j.total == 0) continue;
+      const PairInfo &x = e.pairs[cls[cb][0]], &y = e.pairs[cls[ck][0]];
+      j.g = gradient_class({x.la, x.lb, y.la, y.lb});
+      entries.insert(entries.end(), j.g.entries.begin(), j.g.entries.end());
+      jobs.push_back(std::move(j));
     }
-    // bucket the block tasks by class, row order kept within a class
-    std::vector<size_t> cnt(NKEY + 1, 0);
-    for (int k : rkey) ++cnt[k + 1];
-    for (int k = 0; k < NKEY; ++k) cnt[k + 1] += cnt[k];
-    std::vector<size_t> start(cnt.begin(), cnt.end() - 1);
-    tasks.resize(nbk);
-    for (size_t i = 0; i < nbk; ++i) tasks[cnt[rkey[i]]++] = rtask[i];
-    t_fill += secs(t0, now());
-    const auto t1 = now();
-    if (nbk > cap_t) {
-      d_tasks.alloc(nbk * sizeof(BlockTask));
-      cap_t = nbk;
+  DevBuf d_gp, d_order, d_pre, d_ent, d_tasks, d_blk, d_q;
+  auto up = [&](DevBuf& d, const void* h, size_t bytes) {
+    d.alloc(bytes);
+    HIP_CHECK(hipMemcpyAsync(d.p, h, bytes, hipMemcpyHostToDevice, st));
+  };
+  up(d_gp, gp.data(), gp.size() * sizeof(GPair));
+  up(d_order, order.data(), order.size() * sizeof(int));
+  up(d_pre, pre.data(), pre.size() * sizeof(long long));
+  up(d_ent, entries.data(), entries.size() * sizeof(GEntry));
+  // 128 MB of blocks at a time: they are read back from the last-level cache
+  constexpr long long BUDGET = 1ll << 24;
+  size_t cap_q = 0, cap_t = 0, cap_b = 0;
+  auto batch_of = [&](const Job& j) {
+    long long size = 0;
+    for (int b = 0; b < j.g.blocks.n; ++b) size += j.g.blocks.size[b];
+    const long long most = std::max<long long>(1, std::min<long long>(BUDGET / size, 1 << 19));
+    const long long nq = std::min(j.total, most);
+    cap_q = std::max<size_t>(cap_q, nq);
+    cap_t = std::max<size_t>(cap_t, nq * j.g.blocks.n);
+    cap_b = std::max<size_t>(cap_b, nq * size);
+    return (int)nq;
+  };
+  for (const Job& j : jobs) (void)batch_of(j);
+  d_q.alloc(cap_q * sizeof(int2));
+  d_tasks.alloc(cap_t * sizeof(BlockTask));
+  d_blk.alloc(cap_b * 8);
+  for (Job& j : jobs) {
+    const int most = batch_of(j);
+    GBlocks& g = j.g.blocks;
+    for (long long t0 = 0; t0 < j.total; t0 += most) {
+      const int nq = (int)std::min<long long>(most, j.total - t0);
+      long long base = 0;
+      for (int b = 0; b < g.n; ++b) {
+        g.base[b] = base;
+        base += (long long)nq * g.size[b];
+      }
+      hipLaunchKernelGGL(k_grad_tasks, dim3((nq + 255) / 256), dim3(256), 0, st, d_order.as<int>() + at[j.cb],
+                         d_order.as<int>() + at[j.ck], d_pre.as<long long>() + j.pre, (int)cls[j.cb].size(), t0, nq,
+                         d_gp.as<GPair>(), g, d_q.as<int2>(), d_tasks.as<BlockTask>());
+      HIP_CHECK(hipGetLastError());
+      for (int b = 0; b < g.n; ++b) {
+        const int* k = j.g.key[b];
+        BlockArgs args{d_tasks.as<BlockTask>() + (size_t)b * nq, nq, d_pd.as<PairDev>(), view, e.d_boys.as<double>(),
+                       d_blk.as<double>()};
+        launch_any_block(k[0], k[1], k[2], k[3], args, st);
+      }
+      j.g.c.blocks = g;
+      auto contract = [&](auto gl) {
+        launch_contract<decltype(gl)::value>(j.g.c, d_q.as<int2>(), nq, d_gp.as<GPair>(),
+                                             d_ent.as<GEntry>() + j.entries, d_blk.as<double>(), dP,
+                                             d_scale.as<double>(), n, na, d_grad.as<double>(), st);
+      };
+      const size_t terms = j.g.entries.size();
+      if (terms <= 32)
+        contract(std::integral_constant<int, 4>());
+      else if (terms <= 256)
+        contract(std::integral_constant<int, 16>());
+      else
+        contract(std::integral_constant<int, 64>());
     }
-    if ((size_t)ndbl > cap_b) {
-      d_blk.alloc((size_t)ndbl * 8);
-      cap_b = ndbl;
-    }
-    if (nq > cap_q) {
-      d_q.alloc(nq * sizeof(GQuartet));
-      cap_q = nq;
-    }
-    HIP_CHECK(hipMemcpyAsync(d_tasks.p, tasks.data(), nbk * sizeof(BlockTask), hipMemcpyHostToDevice, st));
-    HIP_CHECK(hipMemcpyAsync(d_q.p, quartets.data(), nq * sizeof(GQuartet), hipMemcpyHostToDevice, st));
-    for (int k = 0; k < NKEY; ++k) {
-      const size_t a0 = start[k], z = cnt[k];  // cnt[k] is now the end of bucket k
-      if (z == a0) continue;
-      BlockArgs args{d_tasks.as<BlockTask>() + a0, (int)(z - a0), d_pd.as<PairDev>(), view, e.d_boys.as<double>(),
-                     d_blk.as<double>()};
-      launch_any_block(k / 125, (k / 25) % 5, (k / 5) % 5, k % 5, args, st);
-    }
-    const int blocks = (int)std::min<size_t>(2048, (nq + 3) / 4);
-    hipLaunchKernelGGL(k_grad_contract, dim3(blocks), dim3(256), lds, st, d_q.as<GQuartet>(), (int)nq,
-                       d_blk.as<double>(), dP, d_scale.as<double>(), n, na, d_grad.as<double>());
-    HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipStreamSynchronize(st));  // the host lists are reused
-    t_gpu += secs(t1, now());
-    ++batches;
   }
-  if (trace)
-    fprintf(stderr, "hfg gradient: %zu pairs, %d batches; count %.3f s, fill %.3f s, device %.3f s, total %.3f s\n",
-            npair, batches, t_count, t_fill, t_gpu, secs(t_start, now()));
   std::vector<double> g2((size_t)3 * na);
   download(g2.data(), d_grad.as<double>(), g2.size(), st);
   for (size_t x = 0; x < g.size(); ++x) grad[x] = g[x] + g2[x];
