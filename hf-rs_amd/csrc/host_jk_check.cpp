@@ -105,7 +105,7 @@ void replay_class_v(Replay& r) {
       const int ket = task.ket0 + lane;
       const ViewDev& vk = P.views[ket];
       const int j = ket - g.start;
-      eri_gc_all<LA, LB, LC, LD, CLS, V>(P.vb.data(), vb.p0, vb.p1, kp, P.kcoef.data() + g.cbase + j, g.base + j,
+      eri_gc_all<LA, LB, LC, LD, CLS, V>(P.vb.data(), vb.p0 + task.pb, vb.p0 + task.pe, kp, P.kcoef.data() + g.cbase + j, g.base + j,
                                       g.npp, g.size, vb.AB, vk.AB,
                                       slice<LA + LB + LC + LD, boys_compact(V, LA + LB + LC + LD)>(), I.data());
       double w = 1.0;
@@ -301,8 +301,8 @@ extern "C" int hfgc_jk_plan_work2(const hfg_basis_view* b, const int* caps, doub
         const ViewDev& vb = plan.views[task.bra];
         const KetGroup& g = plan.groups[task.grp];
         nt += 1;
-        pq += (double)(vb.p1 - vb.p0) * g.npp * task.nket;
-        wave += (double)(vb.p1 - vb.p0) * g.npp;
+        pq += (double)(task.pe - task.pb) * g.npp * task.nket;
+        wave += (double)(task.pe - task.pb) * g.npp;
         at += (double)vb.na * vb.nb * NA * NB;  // bra Coulomb: one per wave
         for (int l = 0; l < task.nket; ++l) {
           const ViewDev& vk = plan.views[task.ket0 + l];

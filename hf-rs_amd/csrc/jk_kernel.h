@@ -205,8 +205,9 @@ __device__ __forceinline__ void jk_task(const MolView& a, double screen0, const 
   const JKTask t = a.tasks[task];
   const int bra = __builtin_amdgcn_readfirstlane(t.bra);
   const int ket0 = __builtin_amdgcn_readfirstlane(t.ket0);
-  int nket = __builtin_amdgcn_readfirstlane(t.nket);
-  const int grp = __builtin_amdgcn_readfirstlane(t.grp);
+  int nket = __builtin_amdgcn_readfirstlane((int)t.nket);
+  const int pb = __builtin_amdgcn_readfirstlane((int)t.pb), pe = __builtin_amdgcn_readfirstlane((int)t.pe);
+  const int grp = __builtin_amdgcn_readfirstlane((int)t.grp);
   if (a.screen > screen0) {
     // A raised threshold (a density change): the task's kets, sorted by
     // bound, keep the prefix with qmax_bra * qmax_ket > screen.
@@ -230,7 +231,7 @@ __device__ __forceinline__ void jk_task(const MolView& a, double screen0, const 
   const KetGroup g = a.groups[grp];
   const int j0 = ket - g.start;
   double I[CA * CC * NBLK];
-  eri_gc<LA, LB, LC, LD, S, V>(a.brec, vb.p0, vb.p1, a.kt, a.kcoef + g.cbase + j0, g.base + j0,
+  eri_gc<LA, LB, LC, LD, S, V>(a.brec, vb.p0 + pb, vb.p0 + pe, a.kt, a.kcoef + g.cbase + j0, g.base + j0,
                          g.npp, g.size, vb.AB, vk.AB, boys, I);  // idle lanes run a valid pair, masked below
 
   double w = 1.0;
@@ -520,18 +521,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
   constexpr int NS = slice_count<LA, LB, LC, LD>();
   constexpr bool BC = boys_compact(V, LA + LB + LC + LD);
   __shared__ double boys[BoysSlice<BC>::size];
-  __shared__ int job_sh;
+  __shared__ int job_sh[2];
   extern __shared__ double rows[];
   // a.nmax is the largest molecule's size: it bounds every job's rows
   for (int e = threadIdx.x; e < NR * a.nmax + CA * NAB; e += blockDim.x) rows[e] = 0.0;
   load_boys_slice<LA + LB + LC + LD, BC>(a.boys, boys);  // ends with a barrier
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
-  for (;;) {
-    if (threadIdx.x == 0) job_sh = atomicAdd(a.job_counter, 1);
-    __syncthreads();
-    const int job = __builtin_amdgcn_readfirstlane(job_sh);
-    __syncthreads();
+  // Job indices alternate between two LDS words.  With many jobs left, the next
+  // one is asked for before the current job's work, so that its round trip to
+  // the counter (one a job: some hundred a workgroup and class on a batch) costs
+  // nothing; towards the end, after it, or a job would wait for a workgroup that
+  // is still at a long one while others are idle ((H2O)4/cc-pVDZ, where most
+  // workgroups have one job: 1.79 ms a build, 2.44 ms with early requests
+  // throughout).
+  if (threadIdx.x == 0) job_sh[0] = atomicAdd(a.job_counter, 1);
+  __syncthreads();
+  for (int turn = 0;; turn ^= 1) {
+    const int job = __builtin_amdgcn_readfirstlane(job_sh[turn]);
     if (job >= a.njob) break;
+    const bool early = a.njob - job > 8 * (int)gridDim.x;
+    int next = 0;
+    if (threadIdx.x == 0 && early) next = atomicAdd(a.job_counter, 1);
     const int de = dir_entry(a.dir_job, a.ndir, job);
     const MolTab* T = a.tabs + ((ciptr)a.dir_mol)[de];
     const MolView m = mol_view(T);
@@ -543,26 +553,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(jk_min_wave
                                           lane, rows);
     }
     __syncthreads();
+    // flush: a wave a row (no division by n per element), the lanes along it
     const ViewDev& vb = m.views[m.tasks[t0].bra];
     const ComboDev* __restrict__ cbra = m.combos + vb.c0;
     const int n = m.n;
-    const int nrow = NR * n + CA * NAB;
     double* __restrict__ Jx = m.Jx;
     double* __restrict__ Kx = m.Kx;
-    for (int e = threadIdx.x; e < nrow; e += blockDim.x) {
-      const double v = rows[e];
-      if (v == 0.0) continue;
-      rows[e] = 0.0;
-      if (e < NR * n) {
-        const int r = e / n, col = e - r * n;
-        const int ao = r < RA * NA ? cbra[(r / NA) * RB].ao_a + r % NA : cbra[(r - RA * NA) / NB].ao_b + (r - RA * NA) % NB;
-        add_local(&Kx[(size_t)ao * n + col], v);
-      } else {
-        const int f = e - NR * n, xy = f / NAB, ij = f % NAB;
-        const int ao_a = cbra[(xy / RB) * RB].ao_a + ij / NB, ao_b = cbra[xy % RB].ao_b + ij % NB;
-        add_local(&Jx[(size_t)ao_a * n + ao_b], v);
+    for (int r = wave; r < NR; r += nwave) {
+      const int ao = __builtin_amdgcn_readfirstlane(r < RA * NA ? cbra[(r / NA) * RB].ao_a + r % NA
+                                                                : cbra[(r - RA * NA) / NB].ao_b + (r - RA * NA) % NB);
+      double* __restrict__ row = rows + (size_t)r * n;
+      double* __restrict__ out = Kx + (size_t)ao * n;
+      for (int col = lane; col < n; col += 64) {
+        const double v = row[col];
+        if (v == 0.0) continue;
+        row[col] = 0.0;
+        add_local(&out[col], v);
       }
     }
+    for (int f = threadIdx.x; f < CA * NAB; f += blockDim.x) {
+      const double v = rows[NR * n + f];
+      if (v == 0.0) continue;
+      rows[NR * n + f] = 0.0;
+      const int xy = f / NAB, ij = f % NAB;
+      const int ao_a = cbra[(xy / RB) * RB].ao_a + ij / NB, ao_b = cbra[xy % RB].ao_b + ij % NB;
+      add_local(&Jx[(size_t)ao_a * n + ao_b], v);
+    }
+    if (threadIdx.x == 0) job_sh[turn ^ 1] = early ? next : atomicAdd(a.job_counter, 1);
     __syncthreads();
   }
 }

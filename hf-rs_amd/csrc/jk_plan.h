@@ -40,10 +40,15 @@ struct ComboDev {
   double q;
 };
 
-// One wave of work: bra view, first ket view and number of ket views (<= 64);
-// all ket views share one primitive count.
+// One wave of work: bra view, first ket view, ket group and number of ket views
+// (<= 64; all share one primitive count), and the range [pb, pe) of the bra
+// view's primitive records it sums over: all of them, or a part (the parts of a
+// quartet's integrals are digested by themselves and add up in J and K).
 struct JKTask {
-  int bra, ket0, nket, grp;
+  int bra, ket0;
+  uint16_t grp;
+  uint8_t nket, pad;
+  uint16_t pb, pe;
 };
 
 // A group of ket views of one pair class, cap and primitive count, contiguous
