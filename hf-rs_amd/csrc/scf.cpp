@@ -174,7 +174,12 @@ static AtomicDensity atomic_hf(const std::vector<Shell>& sh_in, double z) {
   const bool trace = std::getenv("HFG_TRACE") != nullptr;
   const auto t_start = std::chrono::steady_clock::now();
   auto since = [&]() { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count(); };
-  if (!hydrogenic) eng.reset(new Engine(view));
+  if (!hydrogenic) {
+    eng.reset(new Engine(view));
+    // no capture: the solve may run on a set-up thread beside other threads'
+    // allocations and launches
+    eng->use_graph = false;
+  }
   if (trace) std::fprintf(stderr, "[hfg] atomic HF Z=%g n=%d: engine %.4f s\n", z, n, since());
   const size_t nn = (size_t)n * n;
   auto fock = [&](const HMat& P) {
@@ -289,9 +294,20 @@ HMat atomic_density(const std::vector<Shell>& sh, int atom, double z, std::vecto
     if (it != cache.end()) ad = it->second;
   }
   if (ad.p.empty()) {
-    ad = atomic_hf(loc, z);
-    std::lock_guard<std::mutex> lk(mu);
-    cache[key] = ad;
+    // one solve at a time: the set-up threads of a server's first molecules all
+    // ask for the same few atoms at once
+    static std::mutex solve;
+    std::lock_guard<std::mutex> one(solve);
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      auto it = cache.find(key);
+      if (it != cache.end()) ad = it->second;
+    }
+    if (ad.p.empty()) {
+      ad = atomic_hf(loc, z);
+      std::lock_guard<std::mutex> lk(mu);
+      cache[key] = ad;
+    }
   }
   idx.clear();
   for (auto& s : loc)
