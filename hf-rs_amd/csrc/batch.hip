@@ -65,17 +65,21 @@ Fleet::Fleet(int cap) : capacity(cap) {
   d_boys.alloc(tab.size() * sizeof(double));
   HIP_CHECK(hipMemcpyAsync(d_boys.p, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, stream));
   slot_quartets.assign(cap, 0.0);
+  slot_cost.assign(cap, JKClassCost{});
+  if (side_blocks > 0) lanes.reset(new JKLanes(stream));
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
   HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  // Candidates: the default split (the one measured best on (H2O)16/cc-pVDZ),
-  // one stream, only the dp/dd-bra classes aside, the default split with a
-  // larger side grid, only the dd-bra classes aside.
+  // Candidates: four lanes; the split measured best with two streams on
+  // (H2O)16/cc-pVDZ, one stream, only the dp/dd-bra classes aside, the split
+  // with a larger side grid, only the dd-bra classes aside.  The first runs
+  // until the tuner has timed them, and where it never does (a server whose
+  // builds are not all full).
   const unsigned def = default_side_mask();
   unsigned dpdd = 0, dd = 0;
   for (int c = 10; c < HFG_NCLASS; ++c) dpdd |= 1u << c;
   for (int c = 15; c < HFG_NCLASS; ++c) dd |= 1u << c;
-  candidates = {{def, side_blocks, 4}, {def, 0, 4}, {dpdd, side_blocks, 4}, {def, 2 * side_blocks, 4}, {dd, side_blocks / 2, 4}};
+  candidates = {{def, side_blocks, 4, lanes != nullptr}, {def, side_blocks, 4}, {def, 0, 4}, {dpdd, side_blocks, 4}, {def, 2 * side_blocks, 4}, {dd, side_blocks / 2, 4}};
   score.assign(candidates.size(), -1.0);
   const char* at = std::getenv("HFG_AUTOTUNE");
   tuned = side_blocks == 0 || (at && std::atoi(at) == 0);
@@ -104,6 +108,8 @@ void Fleet::attach(int s, const Engine& e, hipStream_t st) {
   tabs[s] = e.tab_host;
   occupied[s] = 1;
   slot_quartets[s] = (double)e.n_quartets;
+  slot_cost[s] = JKClassCost{};
+  slot_cost[s].add(e.plan);
   HIP_CHECK(hipMemcpyAsync(d_tabs.as<MolTab>() + s, &tabs[s], sizeof(MolTab), hipMemcpyHostToDevice, st));
   HIP_CHECK(hipStreamSynchronize(st));  // the host copy may change before the next build
 }
@@ -120,6 +126,9 @@ void Fleet::set_active(const std::vector<int>& slots) {
   }
   active = slots;
   dir = make_directory(slots, th);
+  JKClassCost cost;
+  for (int s : slots) cost.add(slot_cost[s]);
+  assign_lanes(cost, lane);
   if (d_dir.bytes < dir.host.size() * sizeof(int)) d_dir.alloc(std::max<size_t>(dir.host.size(), 1024) * sizeof(int));
   HIP_CHECK(hipMemcpyAsync(d_dir.p, dir.host.data(), dir.host.size() * sizeof(int), hipMemcpyHostToDevice, stream));
   if (!slots.empty())
@@ -143,8 +152,8 @@ void Fleet::tune_step(bool full_build) {
       tuned = true;
       if (std::getenv("HFG_TRACE"))
         for (size_t i = 0; i < score.size(); ++i)
-          fprintf(stderr, "hfg autotune: candidate %zu (side mask %#x, cap %d): %.3e ms/quartet%s\n", i,
-                  candidates[i].side_mask, candidates[i].side_cap, score[i], (int)i == current ? "  <- chosen" : "");
+          fprintf(stderr, "hfg autotune: candidate %zu (%s, side mask %#x, cap %d): %.3e ms/quartet%s\n", i,
+                  candidates[i].four_lanes ? "four lanes" : "side stream", candidates[i].side_mask, candidates[i].side_cap, score[i], (int)i == current ? "  <- chosen" : "");
     } else {
       current = (int)next;
     }
@@ -166,7 +175,13 @@ void Fleet::build(bool full_build) {
   JKLaunch L{d_counters.as<int>(), ev_fork, ev_join, d_boys.as<double>(), screen0, use_rows,
              profile ? events.data() : nullptr, cfg.side_mask, cfg.blocks_per_cu * cus};
   if (pending >= 0) HIP_CHECK(hipEventRecord(tb, stream));
-  launch_jk_set(L, d_tabs.as<MolTab>(), dir, d_dir.as<int>(), stream, side, profile && exclusive ? 0 : cfg.side_cap);
+  if (cfg.four_lanes && !(profile && exclusive)) {
+    int cap[HFG_NCLASS];
+    std::fill(cap, cap + HFG_NCLASS, L.max_blocks);
+    launch_jk_lanes(L, d_tabs.as<MolTab>(), dir, d_dir.as<int>(), lanes->s, lanes->ev, JKLanes::N, lane, cap);
+  } else {
+    launch_jk_set(L, d_tabs.as<MolTab>(), dir, d_dir.as<int>(), stream, side, profile && exclusive ? 0 : cfg.side_cap);
+  }
   if (pending >= 0) HIP_CHECK(hipEventRecord(te, stream));
   if (profile) {
     sync();

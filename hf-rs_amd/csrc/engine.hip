@@ -9,30 +9,33 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <numeric>
 
+#include "block_grid.h"
 #include "engine.h"
 #include "eri_device.h"
+#include "jk_lanes.h"
 #include "orient.h"
 
 namespace hfg {
 
 // One thread per quartet: the unscaled block in kernel orientation.
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(64) void k_block(BlockArgs a) {
+__global__ __launch_bounds__(256) void k_block(BlockArgs a) {
   constexpr int NT = ncart(LA) * ncart(LB) * ncart(LC) * ncart(LD);
   __shared__ double boys[BoysSlice<false>::size];
   load_boys_slice<LA + LB + LC + LD>(a.boys, boys);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.ntask) return;
-  const BlockTask bt = a.tasks[t];
-  const PairDev& pb = a.pairs[bt.bra];
-  const PairDev& pk = a.pairs[bt.ket];
-  double I[NT];
-  eri_block<LA, LB, LC, LD>(a.pp, pb.p0, pb.p1, a.pp, pk.p0, pk.p1 - pk.p0, 1, pb.AB, pk.AB, boys, I);
-  double* o = a.out + bt.off;
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.ntask; t += gridDim.x * blockDim.x) {
+    const BlockTask bt = a.tasks[t];
+    const PairDev& pb = a.pairs[bt.bra];
+    const PairDev& pk = a.pairs[bt.ket];
+    double I[NT];
+    eri_block<LA, LB, LC, LD>(a.pp, pb.p0, pb.p1, a.pp, pk.p0, pk.p1 - pk.p0, 1, pb.AB, pk.AB, boys, I);
+    double* o = a.out + bt.off;
 #pragma unroll
-  for (int i = 0; i < NT; ++i) o[i] = I[i];
+    for (int i = 0; i < NT; ++i) o[i] = I[i];
+  }
 }
 
 __global__ void k_fill(double* p, size_t n, double v);
@@ -160,7 +163,8 @@ static int g_max_blocks = 1024;  // persistent grid: workgroups per launch (set 
 
 template <int LA, int LB, int LC, int LD>
 void launch_block(const BlockArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_block<LA, LB, LC, LD>), dim3((a.ntask + 63) / 64), dim3(64), 0, s, a);
+  const BlockGrid g = block_grid(a.ntask);
+  hipLaunchKernelGGL((k_block<LA, LB, LC, LD>), dim3(g.blocks), dim3(g.threads), 0, s, a);
 }
 
 static const BlockLaunch BLOCK_LAUNCH[HFG_NCLASS_ALL] = {
@@ -504,16 +508,12 @@ void Engine::count_work() {
   }
 }
 
-void launch_jk_set(const JKLaunch& L, const MolTab* d_tabs, const JKDirectory& dr, const int* d_dr, hipStream_t main,
-                   hipStream_t side_stream, int side_cap) {
-  hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, main, L.counters, HFG_NSLOT);
-  // The high-L classes, few and long quartets, run on the side stream with a
-  // capped grid and fill the room the low-L classes leave.
-  auto on_side = [&](int c) { return side_cap > 0 && side_stream && ((L.side_mask >> c) & 1u); };
-  const bool two = side_cap > 0 && side_stream;
-  if (two) {
-    HIP_CHECK(hipEventRecord(L.fork, main));
-    HIP_CHECK(hipStreamWaitEvent(side_stream, L.fork, 0));
+void launch_jk_lanes(const JKLaunch& L, const MolTab* d_tabs, const JKDirectory& dr, const int* d_dr,
+                     const hipStream_t* lanes, const hipEvent_t* ev, int count, const int* lane, const int* cap) {
+  hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, lanes[0], L.counters, HFG_NSLOT);
+  for (int k = 1; k < count; ++k) {
+    HIP_CHECK(hipEventRecord(ev[2 * (k - 1)], lanes[0]));
+    HIP_CHECK(hipStreamWaitEvent(lanes[k], ev[2 * (k - 1)], 0));
   }
   JKArgs a;
   std::memset(&a, 0, sizeof a);
@@ -523,11 +523,11 @@ void launch_jk_set(const JKLaunch& L, const MolTab* d_tabs, const JKDirectory& d
   a.boys = L.boys;
   a.use_rows = L.use_rows ? 1 : 0;
   // A class's two variants run back to back on one stream; its event pair
-  // brackets both.
-  for (int pass = 0; pass < 2; ++pass)
+  // brackets both.  The last lane's classes are issued first.
+  for (int k = count - 1; k >= 0; --k)
     for (int c = 0; c < HFG_NCLASS; ++c) {
-      if ((!dr.count[c] && !dr.count[c + HFG_NCLASS]) || on_side(c) != (pass == 0)) continue;
-      hipStream_t s = on_side(c) ? side_stream : main;
+      if ((!dr.count[c] && !dr.count[c + HFG_NCLASS]) || lane[c] != k) continue;
+      hipStream_t s = lanes[k];
       if (L.events) HIP_CHECK(hipEventRecord(L.events[2 * c], s));
       for (int v = 0; v < 2; ++v) {
         const int slot = c + v * HFG_NCLASS;
@@ -540,14 +540,68 @@ void launch_jk_set(const JKLaunch& L, const MolTab* d_tabs, const JKDirectory& d
         a.njob = dr.njob[slot];
         a.ntask = dr.ntask[slot];
         a.job_counter = L.counters + slot;
-        launch_jk_class(c, v, a, on_side(c) ? side_cap : (L.max_blocks > 0 ? L.max_blocks : g_max_blocks), s);
+        launch_jk_class(c, v, a, cap[c], s);
         HIP_CHECK(hipGetLastError());
       }
       if (L.events) HIP_CHECK(hipEventRecord(L.events[2 * c + 1], s));
     }
-  if (two) {
-    HIP_CHECK(hipEventRecord(L.join, side_stream));
-    HIP_CHECK(hipStreamWaitEvent(main, L.join, 0));
+  for (int k = 1; k < count; ++k) {
+    HIP_CHECK(hipEventRecord(ev[2 * k - 1], lanes[k]));
+    HIP_CHECK(hipStreamWaitEvent(lanes[0], ev[2 * k - 1], 0));
+  }
+}
+
+void launch_jk_set(const JKLaunch& L, const MolTab* d_tabs, const JKDirectory& dr, const int* d_dr, hipStream_t main,
+                   hipStream_t side_stream, int side_cap) {
+  // The high-L classes, few and long quartets, run on the side stream with a
+  // capped grid and fill the room the low-L classes leave.
+  const bool two = side_cap > 0 && side_stream;
+  int lane[HFG_NCLASS], cap[HFG_NCLASS];
+  for (int c = 0; c < HFG_NCLASS; ++c) {
+    lane[c] = two && ((L.side_mask >> c) & 1u) ? 1 : 0;
+    cap[c] = lane[c] ? side_cap : (L.max_blocks > 0 ? L.max_blocks : g_max_blocks);
+  }
+  const hipStream_t lanes[2] = {main, side_stream};
+  const hipEvent_t ev[2] = {L.fork, L.join};
+  launch_jk_lanes(L, d_tabs, dr, d_dr, lanes, ev, two ? 2 : 1, lane, cap);
+}
+
+JKLanes::JKLanes(hipStream_t main) {
+  s[0] = main;
+  for (int k = 1; k < N; ++k) HIP_CHECK(hipStreamCreate(&s[k]));  // default priority
+  for (hipEvent_t& e : ev) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+}
+JKLanes::~JKLanes() {
+  for (int k = 1; k < N; ++k)
+    if (s[k]) (void)hipStreamDestroy(s[k]);
+  for (hipEvent_t e : ev)
+    if (e) (void)hipEventDestroy(e);
+}
+void JKClassCost::add(const JKPlan& plan) {
+  for (int c = 0; c < HFG_NCLASS; ++c)
+    for (size_t j = plan.job_begin[c]; j < plan.job_begin[c + 1]; ++j) {
+      sum[c] += plan.job_cost[j];
+      longest[c] = std::max(longest[c], plan.job_cost[j]);
+    }
+}
+void JKClassCost::add(const JKClassCost& o) {
+  for (int c = 0; c < HFG_NCLASS; ++c) {
+    sum[c] += o.sum[c];
+    longest[c] = std::max(longest[c], o.longest[c]);
+  }
+}
+void assign_lanes(const JKClassCost& cost, int (&lane)[HFG_NCLASS]) {
+  std::array<double, HFG_NCLASS> est;
+  for (int c = 0; c < HFG_NCLASS; ++c)
+    est[c] = cost.sum[c] > 0.0 ? 50.0 + 0.1 / 64.0 * (cost.longest[c] / 4.0 + cost.sum[c] / 2048.0) : 0.0;
+  std::array<int, HFG_NCLASS> by;
+  std::iota(by.begin(), by.end(), 0);
+  std::stable_sort(by.begin(), by.end(), [&](int x, int y) { return est[x] > est[y]; });
+  double load[JKLanes::N] = {};
+  for (int c : by) {
+    const int k = (int)(std::min_element(load, load + JKLanes::N) - load);
+    lane[c] = k;
+    load[k] += est[c];
   }
 }
 
@@ -562,10 +616,19 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
   const size_t nacc = nn * NXCC_SLOTS;
   hipLaunchKernelGGL(k_tab_set, dim3(1), dim3(64), 0, stream, d_tab.as<MolTab>(), dP,
                      dmax > 0.0 && dmax < 1.0 ? screen / dmax : screen);
-  auto launches = [&] {
+  auto launches = [&](const JKLanes* lanes) {
     hipLaunchKernelGGL(k_fill, dim3((nacc + tb - 1) / tb), dim3(tb), 0, stream, d_Jacc.as<double>(), nacc, 0.0);
     hipLaunchKernelGGL(k_fill, dim3((nacc + tb - 1) / tb), dim3(tb), 0, stream, d_Kacc.as<double>(), nacc, 0.0);
-    launch_jk_set(launch_ctx(), d_tab.as<MolTab>(), dir, d_dir.as<int>(), stream, side, side_blocks);
+    if (lanes) {
+      int lane[HFG_NCLASS], cap[HFG_NCLASS];
+      JKClassCost cost;
+      cost.add(plan);
+      assign_lanes(cost, lane);
+      std::fill(cap, cap + HFG_NCLASS, g_max_blocks);
+      launch_jk_lanes(launch_ctx(), d_tab.as<MolTab>(), dir, d_dir.as<int>(), lanes->s, lanes->ev, JKLanes::N, lane,
+                      cap);
+    } else
+      launch_jk_set(launch_ctx(), d_tab.as<MolTab>(), dir, d_dir.as<int>(), stream, side, side_blocks);
     hipLaunchKernelGGL(k_symmetrize, dim3((nn + tb - 1) / tb), dim3(tb), 0, stream, d_Jacc.as<double>(),
                        d_Kacc.as<double>(), dJ, dK, n, dH, dF);
   };
@@ -586,9 +649,12 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
   } else if (g && g->seen >= 1) {
     // second build with these outputs: capture it (the first ran eagerly, so
     // the launch helpers' one-time attribute and occupancy queries are done)
+    // on four lanes, whose streams are only needed for the capture (with one
+    // stream asked for, side_blocks 0, on that one)
+    const std::unique_ptr<JKLanes> lanes(side_blocks > 0 ? new JKLanes(stream) : nullptr);
     HIP_CHECK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
-      launches();
+      launches(lanes.get());
     } catch (...) {
       hipGraph_t partial = nullptr;
       (void)hipStreamEndCapture(stream, &partial);  // leave the stream usable
@@ -601,7 +667,7 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
     HIP_CHECK(hipGraphLaunch(g->exec, stream));
     ++graph_launches;
   } else {
-    launches();
+    launches(nullptr);
     if (g) ++g->seen;
   }
   HIP_CHECK(hipGetLastError());

@@ -17,16 +17,18 @@
 #include <vector>
 
 #include "engine.h"
+#include "jk_lanes.h"
 
 namespace hfg {
 
-// One way to run a build's class launches: which classes go to the side
-// stream (bit mask), that stream's workgroup cap (0: one stream) and the
-// main-stream classes' workgroups per CU.
+// One way to run a build's class launches: over four lanes (jk_lanes.h), or
+// with a side stream: which classes go there (bit mask), its workgroup cap (0:
+// one stream); and the other classes' workgroups per CU.
 struct JKConfig {
   unsigned side_mask;
   int side_cap;
   int blocks_per_cu;
+  bool four_lanes = false;
 };
 
 struct Fleet {
@@ -63,6 +65,9 @@ struct Fleet {
   bool tuned = false;
   hipEvent_t tb = nullptr, te = nullptr;
   std::vector<double> slot_quartets;  // per slot (tuner's work measure)
+  std::vector<JKClassCost> slot_cost;  // per slot
+  std::unique_ptr<JKLanes> lanes;      // null with one stream only (HFG_SIDE_BLOCKS=0)
+  int lane[HFG_NCLASS] = {};           // of the active set's classes
   int cus = 256;
   void tune_step(bool full_build);
   const JKConfig& config() const { return candidates[current]; }

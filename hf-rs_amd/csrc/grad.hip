@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/hfg.h"
+#include "block_grid.h"
 #include "engine.h"
 #include "eri_device.h"
 #include "la_device.h"
@@ -38,25 +39,26 @@ namespace {
 
 // One thread per block, as the engine's block kernels.
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(64) void k_gblock(BlockArgs a) {
+__global__ __launch_bounds__(256) void k_gblock(BlockArgs a) {
   constexpr int NT = ncart(LA) * ncart(LB) * ncart(LC) * ncart(LD);
   __shared__ double boys[BoysSlice<false>::size];
   load_boys_slice<LA + LB + LC + LD>(a.boys, boys);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.ntask) return;
-  const BlockTask bt = a.tasks[t];
-  const PairDev& pb = a.pairs[bt.bra];
-  const PairDev& pk = a.pairs[bt.ket];
-  double I[NT];
-  eri_block<LA, LB, LC, LD>(a.pp, pb.p0, pb.p1, a.pp, pk.p0, pk.p1 - pk.p0, 1, pb.AB, pk.AB, boys, I);
-  double* o = a.out + bt.off;
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.ntask; t += gridDim.x * blockDim.x) {
+    const BlockTask bt = a.tasks[t];
+    const PairDev& pb = a.pairs[bt.bra];
+    const PairDev& pk = a.pairs[bt.ket];
+    double I[NT];
+    eri_block<LA, LB, LC, LD>(a.pp, pb.p0, pb.p1, a.pp, pk.p0, pk.p1 - pk.p0, 1, pb.AB, pk.AB, boys, I);
+    double* o = a.out + bt.off;
 #pragma unroll
-  for (int i = 0; i < NT; ++i) o[i] = I[i];
+    for (int i = 0; i < NT; ++i) o[i] = I[i];
+  }
 }
 
 template <int LA, int LB, int LC, int LD>
 void launch_gblock(const BlockArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_gblock<LA, LB, LC, LD>), dim3((a.ntask + 63) / 64), dim3(64), 0, s, a);
+  const BlockGrid g = block_grid(a.ntask);
+  hipLaunchKernelGGL((k_gblock<LA, LB, LC, LD>), dim3(g.blocks), dim3(g.threads), 0, s, a);
 }
 
 // Rank of a pair class (la >= lb) in the block kernels' order: the orbital
