@@ -24,84 +24,71 @@ struct GemmOp {
   const int* skip;
 };
 
-// 64 x 64 tile of one product per workgroup (grid: N tiles, M tiles, ops):
-// 16 x 16 threads with 4 x 4 outputs each, k panels of 16 staged through LDS
-// in [k][m] / [k][n] order (one padding column against bank conflicts).
+// 32 x 32 tile of one product per workgroup (grid: N tiles, M tiles, ops): each
+// of four waves a 16 x 16 block on the FP64 matrix cores (v_mfma_f64_16x16x4:
+// operands row or column l % 16, contraction index l / 16; result column l % 16,
+// rows l / 16 + 4 r).  The products are small (m 25 to a few hundred) and a
+// purification step waits for each, so what counts is the latency of one tile's
+// chain of k panels: panels 32 wide, the next one on its way to registers during
+// the current one's MFMAs, two LDS buffers, one barrier a panel.  Panels are held
+// [row][k] with a padding column.  Forty def2-SVP molecules: 18.6 us a launch;
+// 67 us with 64 x 64 tiles on the vector units, 16-wide panels loaded after the
+// barrier.
 // Out-of-range tiles of the smaller products of a launch exit at once.
+constexpr int GT = 32, GP = GT + 1;
 __global__ __launch_bounds__(256) inline void k_gemm_batched(const GemmOp* __restrict__ ops) {
+  typedef double d4 __attribute__((ext_vector_type(4)));
   const GemmOp& op = ops[blockIdx.z];
   if (op.skip && *op.skip) return;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  if (m0 >= op.M || n0 >= op.N) return;
-  __shared__ double As[16][65];
-  __shared__ double Bs[16][65];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  double acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
+  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
+  const int M = op.M, N = op.N, K = op.K, lda = op.lda, ldb = op.ldb;
+  if (m0 >= M || n0 >= N) return;
+  __shared__ double As[2][GT * GP], Bs[2][GT * GP];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, lo = t & 31, hi = t >> 5;
   const double* __restrict__ A = op.A;
   const double* __restrict__ B = op.B;
-  for (int k0 = 0; k0 < op.K; k0 += 16) {
+  const bool ta = op.ta, tb = op.tb;
+  double va[4], vb[4];
+  auto load = [&](int k0) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = threadIdx.x + 256 * r;
-      int mm, kk;
-      if (op.ta) {
-        kk = i >> 6;
-        mm = i & 63;
-      } else {
-        mm = i >> 4;
-        kk = i & 15;
-      }
-      const int gm = m0 + mm, gk = k0 + kk;
-      double v = 0.0;
-      if (gm < op.M && gk < op.K) v = op.ta ? A[(size_t)gk * op.lda + gm] : A[(size_t)gm * op.lda + gk];
-      As[kk][mm] = v;
+      const int x = hi + 8 * r;  // consecutive lanes along the stored rows
+      const int am = m0 + (ta ? lo : x), ak = k0 + (ta ? x : lo);
+      va[r] = am < M && ak < K ? A[ta ? (size_t)ak * lda + am : (size_t)am * lda + ak] : 0.0;
+      const int bn = n0 + (tb ? x : lo), bk = k0 + (tb ? lo : x);
+      vb[r] = bn < N && bk < K ? B[tb ? (size_t)bn * ldb + bk : (size_t)bk * ldb + bn] : 0.0;
     }
+  };
+  auto store = [&](int buf) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int i = threadIdx.x + 256 * r;
-      int kk, nn;
-      if (op.tb) {
-        nn = i >> 4;
-        kk = i & 15;
-      } else {
-        kk = i >> 6;
-        nn = i & 63;
-      }
-      const int gk = k0 + kk, gn = n0 + nn;
-      double v = 0.0;
-      if (gk < op.K && gn < op.N) v = op.tb ? B[(size_t)gn * op.ldb + gk] : B[(size_t)gk * op.ldb + gn];
-      Bs[kk][nn] = v;
+      const int x = hi + 8 * r;
+      As[buf][ta ? lo * GP + x : x * GP + lo] = va[r];
+      Bs[buf][tb ? x * GP + lo : lo * GP + x] = vb[r];
     }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      double a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty + 16 * i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
+  };
+  d4 acc = {0.0, 0.0, 0.0, 0.0};
+  const int am = 16 * (w >> 1) + (lane & 15), bn = 16 * (w & 1) + (lane & 15), g = lane >> 4;
+  load(0);
+  store(0);
+  if (K > GT) load(GT);
+  __syncthreads();
+  for (int k0 = 0, buf = 0; k0 < K; k0 += GT, buf ^= 1) {
+    if (k0 + GT < K) {
+      store(buf ^ 1);
+      if (k0 + 2 * GT < K) load(k0 + 2 * GT);
     }
+    const double *a = As[buf] + am * GP + g, *b = Bs[buf] + bn * GP + g;
+#pragma unroll
+    for (int kk = 0; kk < GT; kk += 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[kk], b[kk], acc, 0, 0, 0);
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty + 16 * i;
-    if (gm >= op.M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx + 16 * j;
-      if (gn >= op.N) continue;
-      double* c = op.C + (size_t)gm * op.ldc + gn;
-      *c = op.beta == 0.0 ? op.alpha * acc[i][j] : op.alpha * acc[i][j] + op.beta * *c;
-    }
+  for (int r = 0; r < 4; ++r) {
+    const int gm = m0 + 16 * (w >> 1) + g + 4 * r, gn = n0 + bn;
+    if (gm >= M || gn >= N) continue;
+    double* c = op.C + (size_t)gm * op.ldc + gn;
+    *c = op.beta == 0.0 ? op.alpha * acc[r] : op.alpha * acc[r] + op.beta * *c;
   }
 }
 
@@ -121,8 +108,8 @@ struct GemmList {
     count = (int)ops.size();
     mt = nt = 0;
     for (const GemmOp& o : ops) {
-      mt = std::max(mt, (o.M + 63) / 64);
-      nt = std::max(nt, (o.N + 63) / 64);
+      mt = std::max(mt, (o.M + GT - 1) / GT);
+      nt = std::max(nt, (o.N + GT - 1) / GT);
     }
     if (!count) return;
     if (d_ops.bytes < ops.size() * sizeof(GemmOp)) {
