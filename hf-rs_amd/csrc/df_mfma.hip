@@ -463,31 +463,38 @@ __global__ __launch_bounds__(NT) void k_syrk(const typename T::X* __restrict__ X
   syrk_pick<T, 10>(tl, X, n, k0, k1, lds, part + (size_t)s * n * n);
 }
 
-// K[i][j] = K[j][i] = alpha sum_s part[s][i][j], i <= j, by 32 x 32 tiles (both
-// writes along rows); the sums are in FP64 whatever the partials are.
+// K[i][j] = K[j][i] = alpha sum_s part[s][i][j], i <= j, by 8 x 32 blocks (both
+// writes along rows of a 32 x 32 tile's parts); the sums are in FP64 whatever the
+// partials are, in order, eight loads on their way at a time: one element a
+// thread, since at n = 150 there are 45 blocks of 192 slices (11.5 us; 222 us with
+// 32 x 32 blocks and one load at a time).
 template <class P>
 __global__ __launch_bounds__(256) void k_syrk_reduce(const P* __restrict__ part, int S, int n, double alpha,
                                                      double* __restrict__ K) {
-  __shared__ double tile[32][33];
-  if (blockIdx.y > blockIdx.x) return;
-  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  __shared__ double tile[8][33];
+  const int i0 = blockIdx.y * 8, j0 = blockIdx.x * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+  if (i0 >= j0 + 32) return;
   const size_t nn = (size_t)n * n;
-  for (int r = y; r < 32; r += 8) {
-    const int i = i0 + r, j = j0 + x;
-    double v = 0.0;
-    if (i <= j && j < n) {
-      const P* p = part + (size_t)i * n + j;
-      for (int s = 0; s < S; ++s) v += (double)p[s * nn];
-      v *= alpha;
-      K[(size_t)i * n + j] = v;
+  const int i = i0 + y, j = j0 + x;
+  double v = 0.0;
+  if (i <= j && j < n) {
+    const P* p = part + (size_t)i * n + j;
+    int s = 0;
+    for (; s + 8 <= S; s += 8) {
+      P u[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) u[k] = p[(s + k) * nn];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v += (double)u[k];
     }
-    tile[r][x] = v;
+    for (; s < S; ++s) v += (double)p[s * nn];
+    v *= alpha;
+    K[(size_t)i * n + j] = v;
   }
+  tile[y][x] = v;
   __syncthreads();
-  for (int r = y; r < 32; r += 8) {
-    const int j = j0 + r, i = i0 + x;
-    if (i < j && j < n) K[(size_t)j * n + i] = tile[x][r];
-  }
+  const int c = threadIdx.x & 7, r = threadIdx.x >> 3;  // K[j0 + r][i0 + c]
+  if (i0 + c < j0 + r && j0 + r < n) K[(size_t)(j0 + r) * n + i0 + c] = tile[c][r];
 }
 
 template <class T>
@@ -534,8 +541,8 @@ void k_from_tiles(const double* Bt, size_t npt, int rank, int n, const double* C
   hipLaunchKernelGGL(k_syrk<T>, dim3((unsigned)(tiles * S)), dim3(NT), 0, st, x, n, (int)steps, (int)S, tiles,
                      w.part.template as<P>());
   HIP_CHECK(hipGetLastError());
-  const unsigned g = (unsigned)((n + 31) / 32);
-  hipLaunchKernelGGL(k_syrk_reduce<P>, dim3(g, g), dim3(256), 0, st, w.part.template as<P>(), (int)S, n, 2.0, K);
+  hipLaunchKernelGGL(k_syrk_reduce<P>, dim3((unsigned)((n + 31) / 32), (unsigned)((n + 7) / 8)), dim3(256), 0, st,
+                     w.part.template as<P>(), (int)S, n, 2.0, K);
   HIP_CHECK(hipGetLastError());
 }
 
