@@ -684,12 +684,17 @@ static int df_rhf(const hfg_basis_view* basis, const std::function<DfEngine*()>&
       slot = (int)order.size();
     }
     HIP_CHECK(hipMemcpyAsync(hE.p + (size_t)slot * mm2, dTmp2.p, mm2 * 8, hipMemcpyDeviceToDevice, st));
-    diag(dF.p, dCn.p, dPn.p);
-    hipLaunchKernelGGL(k_sub, grid(nn), dim3(tb), 0, st, dPn.p, dP.p, dTmp.p, nn);
-    const double dch = bl.amax(nn, dTmp.p);
     if (!std::isfinite(ce) || !std::isfinite(resid)) throw HfgError{HFG_INTEGRAL, "DF-HF energy/residual became nonfinite"};
-    if (kprec == 0 && fp64_builds >= 2 && std::fabs(ce - last) <= opt->energy_tol && resid <= opt->residual_tol &&
-        dch <= opt->density_tol) {
+    // the density of F decides convergence only: its eigensolve waits until the
+    // energy and the residual have passed (one eigensolve an iteration instead
+    // of two: the solver was 60 % of a (H2O)6/cc-pVDZ solve)
+    bool done = kprec == 0 && fp64_builds >= 2 && std::fabs(ce - last) <= opt->energy_tol && resid <= opt->residual_tol;
+    if (done) {
+      diag(dF.p, dCn.p, dPn.p);
+      hipLaunchKernelGGL(k_sub, grid(nn), dim3(tb), 0, st, dPn.p, dP.p, dTmp.p, nn);
+      done = bl.amax(nn, dTmp.p) <= opt->density_tol;
+    }
+    if (done) {
       occ_copy(dCn.p);
       fock(dF.p);
       res->total_energy = energy(dPn.p, dF.p) + enuc;
