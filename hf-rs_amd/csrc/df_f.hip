@@ -5,10 +5,13 @@
 // (gen/eri_df.inc), one thread per block as the engine's block kernels, but
 // each block written straight to its output slot: at up to 1,500 doubles a
 // block a private copy would only add scratch.
+#include <map>
+#include <mutex>
 #include <string>
 
 #include "engine.h"
 #include "eri_device.h"
+#include "wide_scratch.h"
 
 namespace hfg {
 #include "gen/eri_df.inc"
@@ -29,11 +32,37 @@ __global__ __launch_bounds__(64) void k_dfblock(BlockArgs a) {
 
 }  // namespace
 
+void launch_wide(hipStream_t s, const std::function<void(hipStream_t)>& launch) {
+  static std::mutex mu;
+  static std::map<int, hipStream_t> streams;  // per device
+  struct Event {
+    hipEvent_t e = nullptr;
+    Event() { HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+    ~Event() { (void)hipEventDestroy(e); }
+  } before, after;
+  int dev = 0;
+  HIP_CHECK(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(mu);
+  hipStream_t& w = streams[dev];
+  if (!w) HIP_CHECK(hipStreamCreate(&w));  // default priority
+  HIP_CHECK(hipEventRecord(before.e, s));
+  HIP_CHECK(hipStreamWaitEvent(w, before.e, 0));
+  launch(w);
+  HIP_CHECK(hipEventRecord(after.e, w));
+  HIP_CHECK(hipStreamWaitEvent(s, after.e, 0));
+}
+
 void launch_df_f_block(int l1, int l2, int l3, int l4, const BlockArgs& a, hipStream_t s) {
 #define X(p, q, r, u)                                                                            \
   if (p == l1 && q == l2 && r == l3 && u == l4) {                                                  \
-    hipLaunchKernelGGL((k_dfblock<p, q, r, u>), dim3((a.ntask + 63) / 64), dim3(64), 0, s, a);      \
-    HIP_CHECK(hipGetLastError());                                                                  \
+    auto launch = [&](hipStream_t on) {                                                            \
+      hipLaunchKernelGGL((k_dfblock<p, q, r, u>), dim3((a.ntask + 63) / 64), dim3(64), 0, on, a);   \
+      HIP_CHECK(hipGetLastError());                                                                \
+    };                                                                                             \
+    if (p + q + r == 10) /* (ff|g): 14,684 bytes a lane */                                         \
+      launch_wide(s, launch);                                                                      \
+    else                                                                                           \
+      launch(s);                                                                                   \
     return;                                                                                        \
   }
   HFG_FOR_EACH_DF_F_CLASS(X)

@@ -25,40 +25,36 @@
 #include <vector>
 
 #include "../../include/hfg.h"
-#include "block_grid.h"
 #include "engine.h"
 #include "eri_device.h"
 #include "la_device.h"
 #include "rhf.h"
 #include "scf_host.h"
+#include "wide_scratch.h"
 
 namespace hfg {
 #include "gen/eri_grad.inc"
 
 namespace {
 
-// One thread per block, as the engine's block kernels.
+// One thread per block, as the engine's block kernels, each block written
+// straight to its place: at up to 2,160 doubles a private copy would only add
+// scratch.
 template <int LA, int LB, int LC, int LD>
-__global__ __launch_bounds__(256) void k_gblock(BlockArgs a) {
-  constexpr int NT = ncart(LA) * ncart(LB) * ncart(LC) * ncart(LD);
+__global__ __launch_bounds__(64) void k_gblock(BlockArgs a) {
   __shared__ double boys[BoysSlice<false>::size];
   load_boys_slice<LA + LB + LC + LD>(a.boys, boys);
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.ntask; t += gridDim.x * blockDim.x) {
-    const BlockTask bt = a.tasks[t];
-    const PairDev& pb = a.pairs[bt.bra];
-    const PairDev& pk = a.pairs[bt.ket];
-    double I[NT];
-    eri_block<LA, LB, LC, LD>(a.pp, pb.p0, pb.p1, a.pp, pk.p0, pk.p1 - pk.p0, 1, pb.AB, pk.AB, boys, I);
-    double* o = a.out + bt.off;
-#pragma unroll
-    for (int i = 0; i < NT; ++i) o[i] = I[i];
-  }
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.ntask) return;
+  const BlockTask bt = a.tasks[t];
+  const PairDev& pb = a.pairs[bt.bra];
+  const PairDev& pk = a.pairs[bt.ket];
+  eri_block<LA, LB, LC, LD>(a.pp, pb.p0, pb.p1, a.pp, pk.p0, pk.p1 - pk.p0, 1, pb.AB, pk.AB, boys, a.out + bt.off);
 }
 
 template <int LA, int LB, int LC, int LD>
 void launch_gblock(const BlockArgs& a, hipStream_t s) {
-  const BlockGrid g = block_grid(a.ntask);
-  hipLaunchKernelGGL((k_gblock<LA, LB, LC, LD>), dim3(g.blocks), dim3(g.threads), 0, s, a);
+  hipLaunchKernelGGL((k_gblock<LA, LB, LC, LD>), dim3((a.ntask + 63) / 64), dim3(64), 0, s, a);
 }
 
 // Rank of a pair class (la >= lb) in the block kernels' order: the orbital
@@ -82,8 +78,14 @@ void launch_any_block(int l1, int l2, int l3, int l4, const BlockArgs& a, hipStr
 #undef X
 #define X(p, q, r, u)                                          \
   if (p == l1 && q == l2 && r == l3 && u == l4) {              \
-    launch_gblock<p, q, r, u>(a, s);                           \
-    HIP_CHECK(hipGetLastError());                              \
+    auto launch = [&](hipStream_t on) {                        \
+      launch_gblock<p, q, r, u>(a, on);                        \
+      HIP_CHECK(hipGetLastError());                            \
+    };                                                         \
+    if (p + q + r + u == 9) /* (fd|dd) */                      \
+      launch_wide(s, launch);                                  \
+    else                                                       \
+      launch(s);                                               \
     return;                                                    \
   }
   HFG_FOR_EACH_GRAD_CLASS(X)
