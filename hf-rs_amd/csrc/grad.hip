@@ -21,6 +21,7 @@
 #include <array>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <type_traits>
 #include <vector>
 
@@ -139,13 +140,14 @@ struct GBlocks {
   int slot[MAX_BLK];   // which of the pair's derivative pairs
   int first[MAX_BLK];  // the block stores the derivative pair first
   int size[MAX_BLK];
-  long long base[MAX_BLK];  // of the block's batch in the block buffer
+  long long base[MAX_BLK];  // of the block's values in the block buffer
+  long long task[MAX_BLK];  // and of its tasks in the task buffer
 };
 
 // Quartet t of a class: rows are the bra class's pairs, each with the prefix of
 // the ket class's pairs (both sorted by Schwarz bound) that passes the test;
 // pre[i] .. pre[i + 1] - 1 are row i's.  Writes the quartet's pairs and its block
-// tasks (block by block, nq each).  One thread a quartet: on the host, listing
+// tasks.  One thread a quartet: on the host, listing
 // the quartets of C8H18/6-31G and copying the lists took 130 of 162 ms; the
 // whole gradient is now 19.4 ms.
 __global__ __launch_bounds__(256) void k_grad_tasks(const int* __restrict__ bra, const int* __restrict__ ket,
@@ -167,7 +169,7 @@ __global__ __launch_bounds__(256) void k_grad_tasks(const int* __restrict__ bra,
   quartets[q] = int2{ij, kl};
   for (int b = 0; b < g.n; ++b) {
     const int dp = pairs[g.ket[b] ? kl : ij].d[g.slot[b]], other = g.ket[b] ? ij : kl;
-    tasks[(size_t)b * nq + q] =
+    tasks[g.task[b] + q] =
         BlockTask{g.first[b] ? dp : other, g.first[b] ? other : dp, g.base[b] + (long long)q * g.size[b]};
   }
 }
@@ -492,50 +494,98 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
   up(d_order, order.data(), order.size() * sizeof(int));
   up(d_pre, pre.data(), pre.size() * sizeof(long long));
   up(d_ent, entries.data(), entries.size() * sizeof(GEntry));
-  // 128 MB of blocks at a time: they are read back from the last-level cache
+  // Rounds of at most 128 MB of blocks (they are read back from the last-level
+  // cache): chunks of one class's quartets, as many as fit, so that a small
+  // molecule's blocks of one kernel go out in one launch whatever classes they
+  // are for (water/6-31G*: 16.8 ms with a round per class).
   constexpr long long BUDGET = 1ll << 24;
-  size_t cap_q = 0, cap_t = 0, cap_b = 0;
-  auto batch_of = [&](const Job& j) {
+  struct Chunk {
+    const Job* job;
+    long long t0;
+    int nq;
+    size_t q0;  // its quartets' place in the round
+    GBlocks g;
+  };
+  struct Launch {
+    const int* key;
+    size_t task0;
+    int count;
+  };
+  struct Round {
+    std::vector<Chunk> chunks;
+    std::vector<Launch> launches;
+    size_t quartets = 0, tasks = 0;
+    long long doubles = 0;
+  };
+  std::vector<Round> rounds(1);
+  for (const Job& j : jobs) {
     long long size = 0;
     for (int b = 0; b < j.g.blocks.n; ++b) size += j.g.blocks.size[b];
-    const long long most = std::max<long long>(1, std::min<long long>(BUDGET / size, 1 << 19));
-    const long long nq = std::min(j.total, most);
-    cap_q = std::max<size_t>(cap_q, nq);
-    cap_t = std::max<size_t>(cap_t, nq * j.g.blocks.n);
-    cap_b = std::max<size_t>(cap_b, nq * size);
-    return (int)nq;
-  };
-  for (const Job& j : jobs) (void)batch_of(j);
+    for (long long t0 = 0; t0 < j.total;) {
+      Round* r = &rounds.back();
+      long long room = std::min<long long>((BUDGET - r->doubles) / size, (1 << 19) - (long long)r->quartets);
+      if (room <= 0 && !r->chunks.empty()) {
+        rounds.emplace_back();
+        r = &rounds.back();
+        room = std::min<long long>(BUDGET / size, 1 << 19);
+      }
+      const int nq = (int)std::min(j.total - t0, std::max<long long>(1, room));
+      Chunk c{&j, t0, nq, r->quartets, j.g.blocks};
+      for (int b = 0; b < c.g.n; ++b) {
+        c.g.base[b] = r->doubles;
+        r->doubles += (long long)nq * c.g.size[b];
+      }
+      r->quartets += nq;
+      r->chunks.push_back(c);
+      t0 += nq;
+    }
+  }
+  size_t cap_q = 0, cap_t = 0, cap_b = 0;
+  for (Round& r : rounds) {
+    std::map<std::array<int, 4>, std::vector<std::pair<Chunk*, int>>> by_key;
+    for (Chunk& c : r.chunks)
+      for (int b = 0; b < c.g.n; ++b) {
+        const int* k = c.job->g.key[b];
+        by_key[{k[0], k[1], k[2], k[3]}].push_back({&c, b});
+      }
+    for (auto& k : by_key) {
+      Launch l{k.second[0].first->job->g.key[k.second[0].second], r.tasks, 0};
+      for (auto& cb : k.second) {
+        cb.first->g.task[cb.second] = (long long)r.tasks;
+        r.tasks += cb.first->nq;
+        l.count += cb.first->nq;
+      }
+      r.launches.push_back(l);
+    }
+    cap_q = std::max(cap_q, r.quartets);
+    cap_t = std::max(cap_t, r.tasks);
+    cap_b = std::max(cap_b, (size_t)r.doubles);
+  }
   d_q.alloc(cap_q * sizeof(int2));
   d_tasks.alloc(cap_t * sizeof(BlockTask));
   d_blk.alloc(cap_b * 8);
-  for (Job& j : jobs) {
-    const int most = batch_of(j);
-    GBlocks& g = j.g.blocks;
-    for (long long t0 = 0; t0 < j.total; t0 += most) {
-      const int nq = (int)std::min<long long>(most, j.total - t0);
-      long long base = 0;
-      for (int b = 0; b < g.n; ++b) {
-        g.base[b] = base;
-        base += (long long)nq * g.size[b];
-      }
-      hipLaunchKernelGGL(k_grad_tasks, dim3((nq + 255) / 256), dim3(256), 0, st, d_order.as<int>() + at[j.cb],
-                         d_order.as<int>() + at[j.ck], d_pre.as<long long>() + j.pre, (int)cls[j.cb].size(), t0, nq,
-                         d_gp.as<GPair>(), g, d_q.as<int2>(), d_tasks.as<BlockTask>());
+  for (const Round& r : rounds) {
+    for (const Chunk& c : r.chunks) {
+      hipLaunchKernelGGL(k_grad_tasks, dim3((c.nq + 255) / 256), dim3(256), 0, st,
+                         d_order.as<int>() + at[c.job->cb], d_order.as<int>() + at[c.job->ck],
+                         d_pre.as<long long>() + c.job->pre, (int)cls[c.job->cb].size(), c.t0, c.nq, d_gp.as<GPair>(),
+                         c.g, d_q.as<int2>() + c.q0, d_tasks.as<BlockTask>());
       HIP_CHECK(hipGetLastError());
-      for (int b = 0; b < g.n; ++b) {
-        const int* k = j.g.key[b];
-        BlockArgs args{d_tasks.as<BlockTask>() + (size_t)b * nq, nq, d_pd.as<PairDev>(), view, e.d_boys.as<double>(),
-                       d_blk.as<double>()};
-        launch_any_block(k[0], k[1], k[2], k[3], args, st);
-      }
-      j.g.c.blocks = g;
+    }
+    for (const Launch& l : r.launches) {
+      BlockArgs args{d_tasks.as<BlockTask>() + l.task0, l.count, d_pd.as<PairDev>(), view, e.d_boys.as<double>(),
+                     d_blk.as<double>()};
+      launch_any_block(l.key[0], l.key[1], l.key[2], l.key[3], args, st);
+    }
+    for (const Chunk& c : r.chunks) {
+      GContract gc = c.job->g.c;
+      gc.blocks = c.g;
       auto contract = [&](auto gl) {
-        launch_contract<decltype(gl)::value>(j.g.c, d_q.as<int2>(), nq, d_gp.as<GPair>(),
-                                             d_ent.as<GEntry>() + j.entries, d_blk.as<double>(), dP,
+        launch_contract<decltype(gl)::value>(gc, d_q.as<int2>() + c.q0, c.nq, d_gp.as<GPair>(),
+                                             d_ent.as<GEntry>() + c.job->entries, d_blk.as<double>(), dP,
                                              d_scale.as<double>(), n, na, d_grad.as<double>(), st);
       };
-      const size_t terms = j.g.entries.size();
+      const size_t terms = c.job->g.entries.size();
       if (terms <= 32)
         contract(std::integral_constant<int, 4>());
       else if (terms <= 256)
