@@ -192,7 +192,9 @@ struct GContract {
 // nine sums and d/dD = -(d/dA + d/dB + d/dC).  GL lanes a quartet, chosen by
 // the class's entries (9 for (ss|ss), 1,197 for (pp|pp)): a wave per quartet
 // had 3 of 64 lanes at work on an (ss|ss) block and formed G again for every
-// entry.  Atoms' forces are summed in LDS per workgroup, then added to grad
+// entry.  The longest lists (17,000 of (dd|dd)) and short launches take a whole
+// workgroup a quartet: a wave's walk through them is what a launch then lasts.
+// Atoms' forces are summed in LDS per workgroup, then added to grad
 // (natom x 3).  w = 1/2 x the quartet's degeneracy.
 template <int GL>
 __global__ __launch_bounds__(256) void k_grad_contract(const int2* __restrict__ quartets, int nq,
@@ -239,10 +241,10 @@ __global__ __launch_bounds__(256) void k_grad_contract(const int2* __restrict__ 
           v += e.coef * blk[c.blocks.base[e.b] + (long long)q * c.blocks.size[e.b] + e.e] * G[e.o];
         }
 #pragma unroll
-      for (int o = GL / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, GL);
+      for (int o = (GL < 64 ? GL : 64) / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, GL < 64 ? GL : 64);
       s[x] = v;
     }
-    if (on && lane == 0) {
+    if (on && lane % 64 == 0) {  // each wave's part, where a quartet has four
       double w = 0.5;
       if (A.ao[0] != A.ao[1]) w *= 2.0;
       if (C.ao[0] != C.ao[1]) w *= 2.0;
@@ -586,12 +588,16 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
                                              d_scale.as<double>(), n, na, d_grad.as<double>(), st);
       };
       const size_t terms = c.job->g.entries.size();
+      // a workgroup a quartet while that leaves CUs idle, or for lists that keep its
+      // 256 lanes busy (and whose G, 10 KB of (dd|dd), limits the quartets on a CU)
       if (terms <= 32)
         contract(std::integral_constant<int, 4>());
       else if (terms <= 256)
         contract(std::integral_constant<int, 16>());
-      else
+      else if (terms <= 4096 && c.nq > 512)
         contract(std::integral_constant<int, 64>());
+      else
+        contract(std::integral_constant<int, 256>());
     }
   }
   std::vector<double> g2((size_t)3 * na);
