@@ -350,6 +350,44 @@ void launch_contract(const GContract& c, const int2* quartets, int nq, const GPa
   HIP_CHECK(hipGetLastError());
 }
 
+// Parts of one device allocation, each from a multiple of 256 bytes, and the host
+// side of those that are copied there in one piece.  add and place come before
+// reserve (no host side), all before upload.
+class Slab {
+ public:
+  size_t place(size_t bytes) {
+    const size_t o = reserve(bytes);
+    host_.resize(size_);
+    return o;
+  }
+  void put(size_t o, const void* h, size_t bytes) {
+    if (bytes) std::memcpy(host_.data() + o, h, bytes);
+  }
+  size_t add(const void* h, size_t bytes) {
+    const size_t o = place(bytes);
+    put(o, h, bytes);
+    return o;
+  }
+  size_t reserve(size_t bytes) {
+    const size_t o = size_;
+    size_ += (bytes + 255) / 256 * 256;
+    return o;
+  }
+  void upload(hipStream_t st) {
+    dev_.alloc(size_);
+    if (!host_.empty()) HIP_CHECK(hipMemcpyAsync(dev_.p, host_.data(), host_.size(), hipMemcpyHostToDevice, st));
+  }
+  template <class T>
+  T* at(size_t o) const {
+    return (T*)((char*)dev_.p + o);
+  }
+
+ private:
+  std::vector<char> host_;
+  size_t size_ = 0;
+  DevBuf dev_;
+};
+
 }  // namespace
 
 // Nuclear gradient (natom x 3, host) of the engine's molecule for the device
@@ -429,20 +467,21 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
     for (int k = 0; k < 3; ++k) d.AB[k] = X.c[k] - Y.c[k];
   }
   const size_t npp = pp.size();
-  DevBuf d_pp, d_pd, d_scale, d_grad;
-  d_pp.alloc(9 * npp * sizeof(double));
-  const std::vector<double>* cols[9] = {&pp.p, &pp.Px, &pp.Py, &pp.Pz, &pp.PAx, &pp.PAy, &pp.PAz, &pp.K, &pp.H};
-  for (int c = 0; c < 9; ++c)
-    HIP_CHECK(hipMemcpyAsync(d_pp.as<double>() + c * npp, cols[c]->data(), npp * 8, hipMemcpyHostToDevice, st));
-  d_pd.alloc(pd.size() * sizeof(PairDev));
-  HIP_CHECK(hipMemcpyAsync(d_pd.p, pd.data(), pd.size() * sizeof(PairDev), hipMemcpyHostToDevice, st));
-  d_scale.alloc((size_t)n * 8);
-  HIP_CHECK(hipMemcpyAsync(d_scale.p, sc.data(), (size_t)n * 8, hipMemcpyHostToDevice, st));
-  d_grad.alloc((size_t)3 * na * 8);
-  hipLaunchKernelGGL(k_zero, dim3((3 * na + 255) / 256), dim3(256), 0, st, d_grad.as<double>(), (size_t)3 * na);
+  // one allocation and one copy for the tables (a small molecule's call is a few
+  // dozen launches of 10 to 50 us: sixteen copies and eleven allocations showed)
+  Slab tables;
+  const size_t o_pp = tables.place(9 * npp * sizeof(double));
+  for (int c = 0; c < 9; ++c) tables.put(o_pp + c * npp * sizeof(double), grow[c]->data(), npp * sizeof(double));
+  const size_t o_pd = tables.add(pd.data(), pd.size() * sizeof(PairDev)), o_scale = tables.add(sc.data(), (size_t)n * 8),
+               o_grad = tables.place((size_t)3 * na * 8);
+  tables.upload(st);
+  double* d_grad = tables.at<double>(o_grad);
+  const PairDev* d_pd = tables.at<PairDev>(o_pd);
+  const double* d_scale = tables.at<double>(o_scale);
+  hipLaunchKernelGGL(k_zero, dim3((3 * na + 255) / 256), dim3(256), 0, st, d_grad, (size_t)3 * na);
   // ---- one-electron terms on the device (onee_dev.hip)
-  onee_gradient_device(sh, n, atoms, dP, dW, d_grad.as<double>(), st);
-  const double* b = d_pp.as<double>();
+  onee_gradient_device(sh, n, atoms, dP, dW, d_grad, st);
+  const double* b = tables.at<double>(o_pp);
   const PrimPairs view{b, b + npp, b + 2 * npp, b + 3 * npp, b + 4 * npp, b + 5 * npp, b + 6 * npp, b + 7 * npp,
                        b + 8 * npp};
   // Quartets by pair of pair classes: both classes' pairs sorted by Schwarz
@@ -487,15 +526,11 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
       entries.insert(entries.end(), j.g.entries.begin(), j.g.entries.end());
       jobs.push_back(std::move(j));
     }
-  DevBuf d_gp, d_order, d_pre, d_ent, d_tasks, d_blk, d_q;
-  auto up = [&](DevBuf& d, const void* h, size_t bytes) {
-    d.alloc(bytes);
-    HIP_CHECK(hipMemcpyAsync(d.p, h, bytes, hipMemcpyHostToDevice, st));
-  };
-  up(d_gp, gp.data(), gp.size() * sizeof(GPair));
-  up(d_order, order.data(), order.size() * sizeof(int));
-  up(d_pre, pre.data(), pre.size() * sizeof(long long));
-  up(d_ent, entries.data(), entries.size() * sizeof(GEntry));
+  Slab lists;
+  const size_t o_gp = lists.add(gp.data(), gp.size() * sizeof(GPair)),
+               o_order = lists.add(order.data(), order.size() * sizeof(int)),
+               o_pre = lists.add(pre.data(), pre.size() * sizeof(long long)),
+               o_ent = lists.add(entries.data(), entries.size() * sizeof(GEntry));
   // Rounds of at most 128 MB of blocks (they are read back from the last-level
   // cache): chunks of one class's quartets, as many as fit, so that a small
   // molecule's blocks of one kernel go out in one launch whatever classes they
@@ -563,29 +598,33 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
     cap_t = std::max(cap_t, r.tasks);
     cap_b = std::max(cap_b, (size_t)r.doubles);
   }
-  d_q.alloc(cap_q * sizeof(int2));
-  d_tasks.alloc(cap_t * sizeof(BlockTask));
-  d_blk.alloc(cap_b * 8);
+  const size_t o_q = lists.reserve(cap_q * sizeof(int2)), o_tasks = lists.reserve(cap_t * sizeof(BlockTask)),
+               o_blk = lists.reserve(cap_b * 8);
+  lists.upload(st);
+  const GPair* d_gp = lists.at<GPair>(o_gp);
+  const int* d_order = lists.at<int>(o_order);
+  const long long* d_pre = lists.at<long long>(o_pre);
+  const GEntry* d_ent = lists.at<GEntry>(o_ent);
+  int2* d_q = lists.at<int2>(o_q);
+  BlockTask* d_tasks = lists.at<BlockTask>(o_tasks);
+  double* d_blk = lists.at<double>(o_blk);
   for (const Round& r : rounds) {
     for (const Chunk& c : r.chunks) {
       hipLaunchKernelGGL(k_grad_tasks, dim3((c.nq + 255) / 256), dim3(256), 0, st,
-                         d_order.as<int>() + at[c.job->cb], d_order.as<int>() + at[c.job->ck],
-                         d_pre.as<long long>() + c.job->pre, (int)cls[c.job->cb].size(), c.t0, c.nq, d_gp.as<GPair>(),
-                         c.g, d_q.as<int2>() + c.q0, d_tasks.as<BlockTask>());
+                         d_order + at[c.job->cb], d_order + at[c.job->ck], d_pre + c.job->pre,
+                         (int)cls[c.job->cb].size(), c.t0, c.nq, d_gp, c.g, d_q + c.q0, d_tasks);
       HIP_CHECK(hipGetLastError());
     }
     for (const Launch& l : r.launches) {
-      BlockArgs args{d_tasks.as<BlockTask>() + l.task0, l.count, d_pd.as<PairDev>(), view, e.d_boys.as<double>(),
-                     d_blk.as<double>()};
+      BlockArgs args{d_tasks + l.task0, l.count, d_pd, view, e.d_boys.as<double>(), d_blk};
       launch_any_block(l.key[0], l.key[1], l.key[2], l.key[3], args, st);
     }
     for (const Chunk& c : r.chunks) {
       GContract gc = c.job->g.c;
       gc.blocks = c.g;
       auto contract = [&](auto gl) {
-        launch_contract<decltype(gl)::value>(gc, d_q.as<int2>() + c.q0, c.nq, d_gp.as<GPair>(),
-                                             d_ent.as<GEntry>() + c.job->entries, d_blk.as<double>(), dP,
-                                             d_scale.as<double>(), n, na, d_grad.as<double>(), st);
+        launch_contract<decltype(gl)::value>(gc, d_q + c.q0, c.nq, d_gp, d_ent + c.job->entries, d_blk, dP,
+                                             d_scale, n, na, d_grad, st);
       };
       const size_t terms = c.job->g.entries.size();
       // a workgroup a quartet while that leaves CUs idle, or for lists that keep its
@@ -601,7 +640,7 @@ void rhf_gradient_device(Engine& e, const std::vector<std::array<double, 4>>& at
     }
   }
   std::vector<double> g2((size_t)3 * na);
-  download(g2.data(), d_grad.as<double>(), g2.size(), st);
+  download(g2.data(), d_grad, g2.size(), st);
   for (size_t x = 0; x < g.size(); ++x) grad[x] = g[x] + g2[x];
 }
 
