@@ -48,7 +48,7 @@ __global__ void k_fleet_jk_out(const MolTab* __restrict__ tabs, const int* __res
   }
 }
 
-Fleet::Fleet(int cap) : capacity(cap) {
+Fleet::Fleet(int cap, bool four_lanes) : capacity(cap) {
   if (cap <= 0) throw HfgError{HFG_INVALID_INPUT, "a fleet needs at least one slot"};
   HIP_CHECK(hipStreamCreate(&stream));  // default priority
   HIP_CHECK(hipStreamCreate(&side));    // default priority
@@ -66,20 +66,23 @@ Fleet::Fleet(int cap) : capacity(cap) {
   HIP_CHECK(hipMemcpyAsync(d_boys.p, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, stream));
   slot_quartets.assign(cap, 0.0);
   slot_cost.assign(cap, JKClassCost{});
-  if (side_blocks > 0) lanes.reset(new JKLanes(stream));
+  if (four_lanes && side_blocks > 0) lanes.reset(new JKLanes(stream));
   int dev = 0;
   HIP_CHECK(hipGetDevice(&dev));
   HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  // Candidates: four lanes; the split measured best with two streams on
-  // (H2O)16/cc-pVDZ, one stream, only the dp/dd-bra classes aside, the split
-  // with a larger side grid, only the dd-bra classes aside.  The first runs
-  // until the tuner has timed them, and where it never does (a server whose
-  // builds are not all full).
+  // Candidates: four lanes, where the fleet has them; the split measured best
+  // with two streams on (H2O)16/cc-pVDZ, one stream, only the dp/dd-bra classes
+  // aside, the split with a larger side grid, only the dd-bra classes aside.
+  // The first runs until the tuner has timed them, and where it never does (a
+  // server whose builds are not all full).
   const unsigned def = default_side_mask();
   unsigned dpdd = 0, dd = 0;
   for (int c = 10; c < HFG_NCLASS; ++c) dpdd |= 1u << c;
   for (int c = 15; c < HFG_NCLASS; ++c) dd |= 1u << c;
-  candidates = {{def, side_blocks, 4, lanes != nullptr}, {def, side_blocks, 4}, {def, 0, 4}, {dpdd, side_blocks, 4}, {def, 2 * side_blocks, 4}, {dd, side_blocks / 2, 4}};
+  if (lanes) candidates.push_back({def, side_blocks, 4, true});
+  for (const JKConfig& c : {JKConfig{def, side_blocks, 4}, {def, 0, 4}, {dpdd, side_blocks, 4}, {def, 2 * side_blocks, 4},
+                            {dd, side_blocks / 2, 4}})
+    candidates.push_back(c);
   score.assign(candidates.size(), -1.0);
   const char* at = std::getenv("HFG_AUTOTUNE");
   tuned = side_blocks == 0 || (at && std::atoi(at) == 0);
@@ -230,7 +233,7 @@ struct Batch {
 
   Batch(const hfg_basis_view* bases, int count) {
     if (count <= 0) throw HfgError{HFG_INVALID_INPUT, "empty batch"};
-    fleet.reset(new Fleet(count));
+    fleet.reset(new Fleet(count, true));
     std::vector<int> slots;
     std::vector<double*> jout, kout;
     for (int m = 0; m < count; ++m) {

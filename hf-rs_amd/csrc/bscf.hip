@@ -547,7 +547,9 @@ struct Server {
 
 Server::Server(const hfg_server_options& o) : opt(o) {
   if (opt.capacity <= 0) throw HfgError{HFG_INVALID_INPUT, "server capacity must be positive"};
-  fleet.reset(new Fleet(opt.capacity));
+  // two streams: a served run that built over four, beside the set-up threads'
+  // own, stopped making progress once; the cause is not known
+  fleet.reset(new Fleet(opt.capacity, false));
   slots.resize(opt.capacity);
   const int cap = opt.capacity;
   d_mols.alloc(cap * sizeof(BMol));

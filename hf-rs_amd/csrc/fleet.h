@@ -21,9 +21,10 @@
 
 namespace hfg {
 
-// One way to run a build's class launches: over four lanes (jk_lanes.h), or
-// with a side stream: which classes go there (bit mask), its workgroup cap (0:
-// one stream); and the other classes' workgroups per CU.
+// One way to run a build's class launches: over four lanes (jk_lanes.h; fleets
+// made with them only), or with a side stream: which classes go there (bit
+// mask), its workgroup cap (0: one stream); and the other classes' workgroups
+// per CU.
 struct JKConfig {
   unsigned side_mask;
   int side_cap;
@@ -66,13 +67,15 @@ struct Fleet {
   hipEvent_t tb = nullptr, te = nullptr;
   std::vector<double> slot_quartets;  // per slot (tuner's work measure)
   std::vector<JKClassCost> slot_cost;  // per slot
-  std::unique_ptr<JKLanes> lanes;      // null with one stream only (HFG_SIDE_BLOCKS=0)
+  std::unique_ptr<JKLanes> lanes;      // null in a server, and with one stream only (HFG_SIDE_BLOCKS=0)
   int lane[HFG_NCLASS] = {};           // of the active set's classes
   int cus = 256;
   void tune_step(bool full_build);
   const JKConfig& config() const { return candidates[current]; }
 
-  explicit Fleet(int capacity);
+  // four_lanes: builds may run over four streams (a batch); a server, whose
+  // set-up threads use streams of their own meanwhile, keeps to two.
+  Fleet(int capacity, bool four_lanes);
   ~Fleet();
   Fleet(const Fleet&) = delete;
   Fleet& operator=(const Fleet&) = delete;

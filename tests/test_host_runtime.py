@@ -1,0 +1,63 @@
+"""The library's host side against a stand-in runtime (hip_stub.cpp): what it does when a device call fails, which
+streams, workspaces and limits it asks for.  Each test runs a short program in a child process with the stand-in
+preloaded; the kernels do nothing there, so only control flow is looked at, never a number."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+HEAD = """
+import ctypes as C, sys, threading
+sys.path.insert(0, {root!r}); sys.path.insert(0, {pkg!r})
+import numpy as np
+import __graft_entry__ as entry
+hf = entry._load()
+import molecules as M
+stub = C.CDLL({stub!r})
+stub.stub_count.restype = C.c_long
+MALLOCS, STREAMS, WATCHED, OUTSIDE, LDS_BEYOND, FAILED, WATCHED_STREAMS = range(7)
+def basis(mol, name):
+    return hf.Basis.from_g94(M.basis_text(name), mol.symbols, mol.xyz)
+def raises(code, call):
+    try:
+        call()
+    except hf.HfError as e:
+        assert e.code == code, (e.code, str(e))
+        return str(e)
+    raise AssertionError("no error")
+water = M.water_config1()
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "hip_stub.cpp")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", so, src, "-lpthread"])
+    head = HEAD.format(root=ROOT, pkg=os.path.join(ROOT, "hf-rs_amd"), stub=so)
+
+    def run(body, **env):
+        pre = os.environ.get("LD_PRELOAD", "")
+        e = dict(os.environ, LD_PRELOAD=(pre + ":" if pre else "") + so, OMP_NUM_THREADS="2", **env)
+        r = subprocess.run([sys.executable, "-c", head + textwrap.dedent(body)], env=e, capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return run
+
+
+def test_server_builds_over_two_streams(program):
+    """The fleet's two and one per set-up worker, and no more when it has run."""
+    program("""
+    srv = hf.Server(capacity=2)
+    assert stub.stub_count(STREAMS) == 2 + 2, stub.stub_count(STREAMS)
+    srv.submit([basis(water, "sto-3g")], [water.zxyz], max_iter=3)
+    srv.run()
+    assert stub.stub_count(STREAMS) == 2 + 2
+    srv.close()
+    assert stub.stub_count(STREAMS) == 0
+    """)
