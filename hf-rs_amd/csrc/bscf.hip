@@ -648,7 +648,8 @@ int Server::admit(int si, int ri, int step, const double* guess, Worker& w) {
     } else {
       try {
         sad_guess_device(s.eng->shells, n, in.atoms, R.charge, s.mol.S, s.mol.P, *w.blas, stq);
-      } catch (HfgError&) {
+      } catch (HfgError& e) {
+        if (e.code == HFG_DEVICE) throw;  // a failed device call fails the request
         core_guess = true;  // src/scf.rs:452-471: core Hamiltonian when SAD is unavailable
       }
     }

@@ -525,7 +525,8 @@ int scf_rhf(const hfg_basis_view* basis, const double* zxyz, int natom, int char
   } else {
     try {
       sad_guess_device(eng.shells, n, atoms, charge, dS.p, dP.p, bl, st);
-    } catch (HfgError&) {
+    } catch (HfgError& e) {
+      if (e.code == HFG_DEVICE) throw;  // a failed device call is no missing guess
       have_sad = false;
     }
   }

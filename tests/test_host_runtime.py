@@ -61,3 +61,25 @@ def test_server_builds_over_two_streams(program):
     srv.close()
     assert stub.stub_count(STREAMS) == 0
     """)
+
+
+@pytest.mark.parametrize("kernel", ["k_sad_scatter", "k_symmetrize"])
+def test_device_errors_of_the_guess_are_reported(program, kernel):
+    """A device call that fails in the SAD guess (its own kernel, or a build of an atomic solve) fails the request or
+    the solve with its message: the core-Hamiltonian start is for a guess that is unavailable, not for one that the
+    device failed to make."""
+    program("""
+    b = basis(water, "sto-3g")
+    stub.stub_fail_kernel(%r)
+    srv = hf.Server(capacity=1)
+    rid = srv.submit([b], [water.zxyz], max_iter=3)
+    srv.run()
+    r = srv.result(rid)
+    assert not r["ok"] and r["status"] == hf.HFG_DEVICE and "stub failure" in r["error"], r
+    if %r == "k_sad_scatter":  # (a solve's own builds use the other one as well)
+        assert "stub failure" in raises(hf.HFG_DEVICE, lambda: hf.scf_rhf(b, water.zxyz, max_iter=3))
+    stub.stub_fail_kernel(b"")
+    again = srv.submit([b], [water.zxyz], max_iter=3)
+    srv.run()
+    assert srv.result(again)["ok"]
+    """ % (kernel.encode(), kernel))
