@@ -674,6 +674,7 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
   if (profile) {
     sync();
     for (int c = 0; c < HFG_NCLASS; ++c) {
+      (void)hipGetLastError();
       if (task_begin[c + 1] == task_begin[c]) continue;
       float ms = 0;
       HIP_CHECK(hipEventElapsedTime(&ms, events[2 * c], events[2 * c + 1]));

@@ -18,8 +18,10 @@ namespace hfg {
 #define RB_CHECK(expr)                                                                   \
   do {                                                                                   \
     rocblas_status _s = (expr);                                                          \
-    if (_s != rocblas_status_success)                                                    \
+    if (_s != rocblas_status_success) {                                                  \
+      (void)hipGetLastError(); /* as HIP_CHECK */                                        \
       throw HfgError{HFG_DEVICE, std::string(#expr) + ": " + rocblas_status_to_string(_s)}; \
+    }                                                                                    \
   } while (0)
 
 

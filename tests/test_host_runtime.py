@@ -83,3 +83,17 @@ def test_device_errors_of_the_guess_are_reported(program, kernel):
     srv.run()
     assert srv.result(again)["ok"]
     """ % (kernel.encode(), kernel))
+
+
+def test_a_reported_error_is_not_reported_again(program):
+    """A failed allocation fails its call with HFG_DEVICE; the runtime keeps the error for the thread's next
+    hipGetLastError, but the next call on another handle of the thread, which succeeds, does not report it."""
+    program("""
+    b = basis(water, "sto-3g")
+    ctx = hf.Context(b)
+    p = np.eye(b.n)
+    ctx.contract_jk(p)
+    stub.stub_fail_malloc(2)
+    raises(hf.HFG_DEVICE, lambda: hf.Context(b))
+    ctx.contract_jk(p)
+    """)
