@@ -525,10 +525,8 @@ struct DfEngine {
   // B_Q . P = 2 sum A_Q . C from its tiles; otherwise it is a pass over B.
   void jk(const double* dC, int o, double* dJ, double* dK, int precision) {
     const size_t nn = (size_t)n * n;
-    if (!d_q.p) {
-      d_q.alloc((size_t)rank * 8);
-      d_tj.alloc(2 * npt * 8);
-    }
+    if (!d_q.p) d_q.alloc((size_t)rank * 8);
+    if (!d_tj.p) d_tj.alloc(2 * npt * 8);  // (its own test: the allocation before may be the one that succeeded)
     double* dq = d_q.as<double>();
     double* tiled_p = d_tj.as<double>();
     double* tiled_j = tiled_p + npt;

@@ -97,3 +97,30 @@ def test_a_reported_error_is_not_reported_again(program):
     raises(hf.HFG_DEVICE, lambda: hf.Context(b))
     ctx.contract_jk(p)
     """)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "bf16x3"])
+def test_df_workspace_after_a_failed_allocation(program, precision):
+    """Every allocation of a first J/K call fails in turn; the next call on the same handle has a whole workspace (J's
+    tiles, the buffer of several that is allocated last, lie in an allocation)."""
+    program("""
+    b, aux = basis(water, "sto-3g"), basis(water, "def2-svp-rifit")
+    c = np.ones((b.n, 5))
+    k = 0
+    while True:
+        k += 1
+        df = hf.DfTensor(b, aux)
+        before = stub.stub_count(FAILED)
+        stub.stub_fail_malloc(k)
+        try:
+            df.jk_precision(c, %r)
+        except hf.HfError as e:
+            assert e.code == hf.HFG_DEVICE
+        if stub.stub_count(FAILED) == before:
+            break
+        stub.stub_watch(b"k_untile_sym", 0)
+        df.jk_precision(c, %r)
+        assert stub.stub_count(WATCHED) == 1 and stub.stub_count(OUTSIDE) == 0, k
+        df.close()
+    assert k > 5
+    """ % (precision, precision))
