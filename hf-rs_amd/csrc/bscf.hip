@@ -432,7 +432,6 @@ struct Slot {
   int n = 0, m = 0, nocc = 0, elen = 0;
   double enuc = 0;
   DevBuf mem;        // every matrix of the slot, carved by layout()
-  size_t cap = 0;    // doubles held by mem
   size_t footprint = 0;
   BMol mol{};
   // iteration state (scf.cpp's loop variables)
@@ -459,7 +458,7 @@ static size_t slot_doubles(int n, int m) { return slot_layout(n, m, nullptr); }
 static void layout(Slot& s) {
   size_t off[SM_COUNT];
   const size_t total = slot_layout(s.n, s.m, off);
-  if (total > s.cap) throw HfgError{HFG_DEVICE, "slot buffer smaller than its layout"};
+  if (total * sizeof(double) > s.mem.bytes) throw HfgError{HFG_DEVICE, "slot buffer smaller than its layout"};
   double* p = s.mem.as<double>();
   BMol& M = s.mol;
   M.n = s.n;
@@ -628,11 +627,8 @@ int Server::admit(int si, int ri, int step, const double* guess, Worker& w) {
     s.m = orthogonalizer(*w.blas, stq, s.eng->shells, n, dS.p, R.opt.spherical != 0, X);
     if (s.nocc > s.m) throw HfgError{HFG_INVALID_INPUT, "more occupied orbitals than retained overlap rank"};
     s.elen = s.m < n ? s.m * s.m : (int)nn;
-    const size_t need = slot_doubles(n, s.m);
-    if (need > s.cap) {
-      s.mem.alloc(need * sizeof(double));
-      s.cap = need;
-    }
+    const size_t need = slot_doubles(n, s.m) * sizeof(double);
+    if (need > s.mem.bytes) s.mem.alloc(need);
     layout(s);
     HIP_CHECK(hipMemcpyAsync(s.mol.S, dS.p, nn * 8, hipMemcpyDeviceToDevice, stq));
     HIP_CHECK(hipMemcpyAsync(s.mol.H, dH.p, nn * 8, hipMemcpyDeviceToDevice, stq));

@@ -124,3 +124,31 @@ def test_df_workspace_after_a_failed_allocation(program, precision):
         df.close()
     assert k > 5
     """ % (precision, precision))
+
+
+def test_server_slot_after_a_failed_allocation(program):
+    """Every allocation of the set-up of a larger molecule fails in turn; the smaller one that takes the slot next has
+    a buffer (its density lies in an allocation)."""
+    program("""
+    small, large = basis(water, "sto-3g"), basis(water, "cc-pvdz")
+    k = hit = 0
+    while True:
+        k += 1
+        srv = hf.Server(capacity=1)
+        first = srv.submit([small], [water.zxyz], max_iter=2)
+        srv.run()
+        srv.submit([large], [water.zxyz], max_iter=2)
+        before = stub.stub_count(FAILED)
+        stub.stub_watch(b"k_clear", 0)
+        stub.stub_fail_malloc(k)
+        try:
+            srv.run()  # the larger one first, then the smaller one again
+        except hf.HfError as e:
+            assert e.code == hf.HFG_DEVICE
+        assert stub.stub_count(OUTSIDE) == 0, k
+        stub.stub_fail_malloc(0)
+        srv.close()
+        if stub.stub_count(FAILED) == before or k == 60:
+            break
+    assert k > 20
+    """)
