@@ -79,6 +79,10 @@ JKDirectory make_directory(const std::vector<int>& mol, const std::vector<const 
 // shell) with at most max_blocks workgroups; the kernels are split over five
 // translation units.
 void launch_jk_class(int cls, int v, const JKArgs& a, int max_blocks, hipStream_t s);
+// Lets the kernel ask for bytes of dynamic LDS on device dev.  The limit is the
+// kernel's, not the calling thread's: it is only ever raised, so that no thread
+// takes back what another's launches rely on.
+void raise_dynamic_lds(const void* kernel, int dev, size_t bytes);
 // Whether class cls runs on the side stream: (ds|ds) and the classes with a dp
 // or dd bra, (dp|ss) .. (dd|dd), unless HFG_SIDE_CLASSES lists class indices
 // (comma-separated; measured on (H2O)16/cc-pVDZ).

@@ -3,14 +3,18 @@
 // shell blocks, the packed tensor and the density-fitting integrals) and the
 // Fock-build driver over the J/K kernels (jk_kernel.h, jk_plan.cpp).
 #include <algorithm>
+#include <atomic>
 #include <array>
 #include <chrono>
 #include <cstdio>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <memory>
+#include <mutex>
 #include <numeric>
+#include <utility>
 
 #include "block_grid.h"
 #include "engine.h"
@@ -159,7 +163,7 @@ bool side_class(int cls) { return cls >= 0 && cls < HFG_NCLASS && ((default_side
 // ---------------------------------------------------------------------------
 typedef void (*BlockLaunch)(const BlockArgs&, hipStream_t);
 
-static int g_max_blocks = 1024;  // persistent grid: workgroups per launch (set from the CU count)
+static std::atomic<int> g_max_blocks{1024};  // persistent grid: workgroups per launch (set from the CU count)
 
 template <int LA, int LB, int LC, int LD>
 void launch_block(const BlockArgs& a, hipStream_t s) {
@@ -213,8 +217,9 @@ Engine::Engine(const hfg_basis_view& b, hipStream_t shared) {
   {
     int cus = 0;
     HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-    g_max_blocks = std::max(1, cus) * 4;  // 4 workgroups (16 waves) per CU; LDS 4 x 32 KB
-    if (const char* env = std::getenv("HFG_PERSISTENT_BLOCKS")) g_max_blocks = std::max(1, std::atoi(env));
+    int blocks = std::max(1, cus) * 4;  // 4 workgroups (16 waves) per CU; LDS 4 x 32 KB
+    if (const char* env = std::getenv("HFG_PERSISTENT_BLOCKS")) blocks = std::max(1, std::atoi(env));
+    g_max_blocks = blocks;
   }
   build_pairs(shells, pairs, pp);
   ao_scale.assign(n, 1.0);
@@ -559,7 +564,7 @@ void launch_jk_set(const JKLaunch& L, const MolTab* d_tabs, const JKDirectory& d
   int lane[HFG_NCLASS], cap[HFG_NCLASS];
   for (int c = 0; c < HFG_NCLASS; ++c) {
     lane[c] = two && ((L.side_mask >> c) & 1u) ? 1 : 0;
-    cap[c] = lane[c] ? side_cap : (L.max_blocks > 0 ? L.max_blocks : g_max_blocks);
+    cap[c] = lane[c] ? side_cap : (L.max_blocks > 0 ? L.max_blocks : g_max_blocks.load());
   }
   const hipStream_t lanes[2] = {main, side_stream};
   const hipEvent_t ev[2] = {L.fork, L.join};
@@ -605,6 +610,16 @@ void assign_lanes(const JKClassCost& cost, int (&lane)[HFG_NCLASS]) {
   }
 }
 
+void raise_dynamic_lds(const void* kernel, int dev, size_t bytes) {
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, size_t> limit;
+  std::lock_guard<std::mutex> lk(mu);
+  size_t& have = limit[{kernel, dev}];
+  if (bytes <= have) return;
+  HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  have = bytes;
+}
+
 JKLaunch Engine::launch_ctx() {
   return JKLaunch{d_counters.as<int>(), ev_fork, ev_join, d_boys.as<double>(), screen, use_rows,
                   profile ? events.data() : nullptr, default_side_mask(), 0};
@@ -624,7 +639,7 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
       JKClassCost cost;
       cost.add(plan);
       assign_lanes(cost, lane);
-      std::fill(cap, cap + HFG_NCLASS, g_max_blocks);
+      std::fill(cap, cap + HFG_NCLASS, g_max_blocks.load());
       launch_jk_lanes(launch_ctx(), d_tab.as<MolTab>(), dir, d_dir.as<int>(), lanes->s, lanes->ev, JKLanes::N, lane,
                       cap);
     } else
@@ -659,6 +674,7 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
       hipGraph_t partial = nullptr;
       (void)hipStreamEndCapture(stream, &partial);  // leave the stream usable
       if (partial) (void)hipGraphDestroy(partial);
+      (void)hipGetLastError();
       use_graph = false;
       throw;
     }
@@ -674,7 +690,6 @@ void Engine::jk_device(const double* dP, double* dJ, double* dK, const double* d
   if (profile) {
     sync();
     for (int c = 0; c < HFG_NCLASS; ++c) {
-      (void)hipGetLastError();
       if (task_begin[c + 1] == task_begin[c]) continue;
       float ms = 0;
       HIP_CHECK(hipEventElapsedTime(&ms, events[2 * c], events[2 * c + 1]));

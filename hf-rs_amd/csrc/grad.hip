@@ -341,9 +341,11 @@ void launch_contract(const GContract& c, const int2* quartets, int nq, const GPa
                      const double* blk, const double* P, const double* scale, int n, int natom, double* grad,
                      hipStream_t st) {
   const size_t lds = (3 * (size_t)natom + (size_t)(256 / GL) * c.dim[0] * c.dim[1] * c.dim[2] * c.dim[3]) * 8;
-  if (lds > 65536)
-    HIP_CHECK(hipFuncSetAttribute((const void*)k_grad_contract<GL>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)lds));
+  if (lds > 65536) {
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    raise_dynamic_lds((const void*)k_grad_contract<GL>, dev, lds);
+  }
   const int blocks = std::min(2048, (nq + 256 / GL - 1) / (256 / GL));
   hipLaunchKernelGGL(k_grad_contract<GL>, dim3(blocks), dim3(256), lds, st, quartets, nq, pairs, c, entries, blk, P,
                      scale, n, natom, grad);

@@ -612,8 +612,7 @@ void launch_jk(const JKArgs& a, int max_blocks, hipStream_t s) {
   if (a.use_rows && a.njob > 0 && lds + sizeof(double) * BoysSlice<boys_compact(V, LA + LB + LC + LD)>::size + 64 <= (size_t)lds_limit) {
     if (lds != cached_lds) {
       int per_cu = 0;
-      HIP_CHECK(hipFuncSetAttribute((const void*)k_jk_rows<LA, LB, LC, LD, V>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      raise_dynamic_lds((const void*)k_jk_rows<LA, LB, LC, LD, V>, dev, lds);
       HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_jk_rows<LA, LB, LC, LD, V>,
                                                              64 * waves_per_block, lds));
       resident = std::max(1, per_cu) * cus;

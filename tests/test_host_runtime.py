@@ -152,3 +152,20 @@ def test_server_slot_after_a_failed_allocation(program):
             break
     assert k > 20
     """)
+
+
+def test_lds_limit_of_a_kernel_is_shared_by_the_threads(program):
+    """The limit that a kernel's launches with much LDS rely on is the kernel's: another thread's builds of a smaller
+    molecule leave it, so that no launch asks for more than is allowed."""
+    program("""
+    small, large = basis(water, "sto-3g"), basis(M.water_cluster_m(6, 1), "6-31g*")
+    a = hf.Context(large)
+    a.contract_jk(np.eye(large.n))
+    def other():
+        hf.Context(small).contract_jk(np.eye(small.n))
+    t = threading.Thread(target=other)
+    t.start(); t.join()
+    for _ in range(2):
+        a.contract_jk(np.eye(large.n))
+    assert stub.stub_count(LDS_BEYOND) == 0, stub.stub_count(LDS_BEYOND)
+    """)
