@@ -104,20 +104,20 @@ void launch_block_class(int cls, const BlockArgs& a, hipStream_t s);
 // The 3-index classes with an orbital f-p, f-d or f-f pair (df_f.hip).
 void launch_df_f_block(int l1, int l2, int l3, int l4, const BlockArgs& a, hipStream_t s);
 
+// The runtime also keeps a failed call's error for the thread's next
+// hipGetLastError, however many calls succeed before it; thrown, it is taken
+// from there, or the next launch's check would report it again.
 #define HIP_CHECK(expr)                                                                           \
   do {                                                                                            \
     hipError_t _e = (expr);                                                                       \
     if (_e != hipSuccess) {                                                                       \
       (void)hipGetLastError();                                                                    \
-// The runtime also keeps a failed call's error for the thread's next
-// hipGetLastError, however many calls succeed before it; thrown, it is taken
-// from there, or the next launch's check would report it again.
       throw ::hfg::HfgError{HFG_DEVICE, std::string(#expr) + ": " + hipGetErrorString(_e)};     \
+    }                                                                                             \
   } while (0)
 
 struct DevBuf {
   void* p = nullptr;
-    }                                                                                             \
   size_t bytes = 0;
   void alloc(size_t b) {
     free();
