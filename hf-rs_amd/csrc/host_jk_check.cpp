@@ -6,9 +6,13 @@
 // per-combination Schwarz test.  Not part of libhfg.so; never a fallback.
 #define HFG_HOST_CHECK 1
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "classes.h"
 #include "eri_device.h"
@@ -88,6 +92,9 @@ void eri_gc_all(const double* br, int b0, int b1, const PrimPairs& kp, const dou
 
 // The class's tasks evaluated with the kernels' generated recurrences of
 // variant V and digested element by element.
+// First record past those that a task sums over.
+int records_end(const JKTask& t, const ViewDev& vb) { return t.pe == JKTask::ALL ? vb.p1 : vb.p0 + t.pe; }
+
 template <int LA, int LB, int LC, int LD, int CLS, int V>
 void replay_class_v(Replay& r) {
   constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
@@ -105,7 +112,7 @@ void replay_class_v(Replay& r) {
       const int ket = task.ket0 + lane;
       const ViewDev& vk = P.views[ket];
       const int j = ket - g.start;
-      eri_gc_all<LA, LB, LC, LD, CLS, V>(P.vb.data(), vb.p0 + task.pb, vb.p0 + task.pe, kp, P.kcoef.data() + g.cbase + j, g.base + j,
+      eri_gc_all<LA, LB, LC, LD, CLS, V>(P.vb.data(), vb.p0 + task.pb, records_end(task, vb), kp, P.kcoef.data() + g.cbase + j, g.base + j,
                                       g.npp, g.size, vb.AB, vk.AB,
                                       slice<LA + LB + LC + LD, boys_compact(V, LA + LB + LC + LD)>(), I.data());
       double w = 1.0;
@@ -301,8 +308,8 @@ extern "C" int hfgc_jk_plan_work2(const hfg_basis_view* b, const int* caps, doub
         const ViewDev& vb = plan.views[task.bra];
         const KetGroup& g = plan.groups[task.grp];
         nt += 1;
-        pq += (double)(task.pe - task.pb) * g.npp * task.nket;
-        wave += (double)(task.pe - task.pb) * g.npp;
+        pq += (double)(records_end(task, vb) - vb.p0 - task.pb) * g.npp * task.nket;
+        wave += (double)(records_end(task, vb) - vb.p0 - task.pb) * g.npp;
         at += (double)vb.na * vb.nb * NA * NB;  // bra Coulomb: one per wave
         for (int l = 0; l < task.nket; ++l) {
           const ViewDev& vk = plan.views[task.ket0 + l];
@@ -379,5 +386,44 @@ extern "C" int hfgc_jk_plan_jobs(const hfg_basis_view* b, double* out) {
   } catch (std::exception& e) {
     g_err = e.what();
     return 1;
+  }
+}
+
+// The plan with every bound taken as 1 (nothing screened out, nothing evaluated): out[0] = tasks, out[1] = quartet
+// chunks whose tasks' record ranges do not tile the bra view's records exactly once, out[2] = the longest range.
+extern "C" int hfgc_jk_plan_ranges(const hfg_basis_view* b, long long* out) {
+  try {
+    const std::vector<Shell> sh = group_shells(*b);
+    const size_t npair = sh.size() * (sh.size() + 1) / 2;
+    BlockFn ones = [](const PrimPairHost&, const std::vector<PairDev>&, const std::vector<BlockTask>&,
+                      const std::vector<int>&, std::vector<double>& o) { std::fill(o.begin(), o.end(), 1.0); };
+    const JKPlan plan = make_jk_plan(sh, std::vector<double>(npair, 1.0), std::vector<double>(b->n_functions, 1.0),
+                                     1e-12, 1e-20, ones);
+    out[0] = (long long)plan.tasks.size();
+    out[1] = out[2] = 0;
+    for (int c = 0; c < HFG_NCLASS; ++c) {
+      std::map<std::array<int, 3>, std::vector<std::pair<int, int>>> parts;  // (bra, first ket, group)
+      for (size_t t = plan.task_begin[c]; t < plan.task_begin[c + 1]; ++t) {
+        const JKTask& k = plan.tasks[t];
+        const ViewDev& v = plan.views[k.bra];
+        parts[{k.bra, k.ket0, k.grp}].push_back({k.pb, records_end(k, v) - v.p0});
+        out[2] = std::max<long long>(out[2], parts[{k.bra, k.ket0, k.grp}].back().second - k.pb);
+      }
+      for (auto& p : parts) {
+        std::sort(p.second.begin(), p.second.end());
+        int at = 0;
+        bool ok = true;
+        for (const auto& r : p.second) {
+          ok = ok && r.first == at && r.second > r.first;
+          at = r.second;
+        }
+        const ViewDev& v = plan.views[p.first[0]];
+        if (!ok || at != v.p1 - v.p0) ++out[1];
+      }
+    }
+    return 0;
+  } catch (HfgError& e) {
+    g_err = e.msg;
+    return e.code;
   }
 }

@@ -231,7 +231,7 @@ __device__ __forceinline__ void jk_task(const MolView& a, double screen0, const 
   const KetGroup g = a.groups[grp];
   const int j0 = ket - g.start;
   double I[CA * CC * NBLK];
-  eri_gc<LA, LB, LC, LD, S, V>(a.brec, vb.p0 + pb, vb.p0 + pe, a.kt, a.kcoef + g.cbase + j0, g.base + j0,
+  eri_gc<LA, LB, LC, LD, S, V>(a.brec, vb.p0 + pb, pe == JKTask::ALL ? vb.p1 : vb.p0 + pe, a.kt, a.kcoef + g.cbase + j0, g.base + j0,
                          g.npp, g.size, vb.AB, vk.AB, boys, I);  // idle lanes run a valid pair, masked below
 
   double w = 1.0;

@@ -451,10 +451,8 @@ JKPlan make_jk_plan(const std::vector<Shell>& shells, const std::vector<double>&
   }
 
   lap("tables");
-  // a task holds its group and its record range in 16 bits each
+  // (groups of one set differ in primitive count: as many would hold some 200 million records)
   if (groups.size() > 65535) throw HfgError{HFG_UNSUPPORTED, "J/K plan: too many ket groups"};
-  for (const ViewDev& v : vd)
-    if (v.p1 - v.p0 > 65535) throw HfgError{HFG_UNSUPPORTED, "J/K plan: too many primitive pairs in one shell pair"};
   // ---- tasks per class: bra views of the class's bra set, ket groups of its
   // ket set; kets with qmax_bra * qmax_ket > screen form a prefix.  When bra
   // and ket sets coincide each unordered pair of views is listed once.  The
@@ -533,11 +531,12 @@ JKPlan make_jk_plan(const std::vector<Shell>& shells, const std::vector<double>&
         const ViewDev& vb = vd[whole[t].bra];
         const int np = vb.p1 - vb.p0;
         const double steps = (double)np * kg[whole[t].grp].npp;
-        const int parts = std::max(1, std::min(np, (int)(steps / grain)));
+        const bool cut = np < JKTask::ALL;
+        const int parts = cut ? std::max(1, std::min(np, (int)(steps / grain))) : 1;
         for (int q = 0; q < parts; ++q) {
           tl.push_back(whole[t]);
           tl.back().pb = (uint16_t)((long long)np * q / parts);
-          tl.back().pe = (uint16_t)((long long)np * (q + 1) / parts);
+          tl.back().pe = (uint16_t)(cut ? (long long)np * (q + 1) / parts : JKTask::ALL);
         }
         cost += whole[t].nket * (steps + parts * digest);
       }

@@ -152,6 +152,23 @@ def test_kernel_boys_path_between_grid_rows(compact):
     assert worst < 1e-14, worst
 
 
+@pytest.mark.parametrize("lengths", [(3, 2), (81, 81), (256, 255), (256, 256), (300, 7)])
+def test_jk_tasks_tile_the_primitive_pairs(lengths):
+    """Two s shells of the given contraction lengths: the tasks of every
+    quartet chunk cover the bra view's primitive pairs once, also beyond
+    65,535 of them (256 x 256) in one shell pair."""
+    L = cpucheck()
+    L.hfgc_jk_last_error.restype = C.c_char_p
+    k1, k2 = lengths
+    e = [np.geomspace(0.05, 500.0, k) for k in (k1, k2)]
+    arr = [np.array([0, 1], np.int32), np.array([0.0, 0, 0, 0, 0, 1.4]), np.zeros(6, np.int32),
+           np.array([0, k1, k1 + k2], np.int32), np.concatenate(e), np.full(k1 + k2, 0.1)]
+    v = View(2, *[a.ctypes.data for a in arr])
+    out = np.zeros(3, np.int64)
+    assert L.hfgc_jk_plan_ranges(C.byref(v), out.ctypes.data_as(C.c_void_p)) == 0, L.hfgc_jk_last_error()
+    assert out[0] >= 3 and out[1] == 0 and out[2] <= k1 * max(k1, k2), out
+
+
 @pytest.mark.parametrize("basis,cells", [("sto-3g", (2, 1, 1)), ("6-31g*", (2, 1, 1)), ("cc-pvdz", (2, 1, 1)),
                                          ("def2-svp", (2, 1, 1)), ("cc-pvdz", (2, 2, 1))])
 def test_jk_plan_replay_matches_oracle(basis, cells):
