@@ -218,6 +218,11 @@ struct DfEngine {
   DevBuf d_io;  // J, K and C of a call with host buffers
   ExchangeWork xwork;
   static constexpr size_t T_CHUNK = 8ull << 30;  // bytes of one column chunk of the 3-index tensor
+  // HFG_DF_CHUNK: smaller ones (one tile row at least)
+  static size_t chunk_bytes() {
+    const char* e = std::getenv("HFG_DF_CHUNK");
+    return e ? std::min<size_t>(T_CHUNK, std::strtoull(e, nullptr, 10)) : T_CHUNK;
+  }
 
   DfEngine(const hfg_basis_view& basis, const hfg_basis_view& auxv, double cutoff) {
     if (!(cutoff > 0) || !std::isfinite(cutoff))
@@ -428,11 +433,12 @@ struct DfEngine {
     // follow from one GEMM, so the tensor never exists whole.  A shell pair
     // whose functions lie in two chunks is evaluated for both.
     const int nt = tiles_of(n);
+    const double chunk_max = (double)chunk_bytes();
     auto tiles_before = [](int I) { return (size_t)I * (I + 1) / 2; };
     std::vector<std::pair<int, int>> rows;  // chunks of tile rows
     for (int I = 0; I < nt;) {
       int e = I + 1;
-      while (e < nt && 8.0 * naux * (tiles_before(e + 1) - tiles_before(I)) * (TL * TL) <= (double)T_CHUNK) ++e;
+      while (e < nt && 8.0 * naux * (tiles_before(e + 1) - tiles_before(I)) * (TL * TL) <= chunk_max) ++e;
       rows.push_back({I, e});
       I = e;
     }

@@ -1,7 +1,8 @@
 """The matrix-core exchange products over the tiled factor (coulomb_exchange_rhf,
 src/df.rs:133-174) at the sizes where their tiles end: molecules whose n lies
-below, at and above multiples of the 32-wide factor tiles and the 128-row
-output tiles, and column counts around the 16-column blocks and the 160
+below, at and above multiples of the 32-wide factor tiles and the 64-row
+output tiles, with one, two and three column tiles (of at most 160) to the
+first row of them, and column counts around the 16-column blocks and the 160
 columns of one workgroup.
 
 Two references.  The oracle's B gives J and K to 1e-9 per element (the
@@ -37,22 +38,45 @@ MOLECULES = {"water_sto3g": (M.water_config1, "sto-3g"), "water_ccpvdz": (M.wate
 AUX = "def2-svp-rifit"
 
 
-@pytest.fixture(scope="module", params=sorted(MOLECULES))
-def system(hf, request):
-    make, basis = MOLECULES[request.param]
+# n: 175 and 325, two and three column tiles
+LARGE = {"water7_ccpvdz": (lambda: M.water_cluster_m(7, 1), "cc-pvdz"),
+         "water13_ccpvdz": (lambda: M.water_cluster_m(13, 1), "cc-pvdz")}
+
+
+def factors(hf, make, basis):
     mol = make()
     b = hf.Basis.from_g94(M.basis_text(basis), mol.symbols, mol.xyz)
     a = hf.Basis.from_g94(M.basis_text(AUX), mol.symbols, mol.xyz)
-    df = hf.DfTensor(b, a)
-    bt = O.df_build(O.Basis.build(M.basis_text(basis), mol.symbols, mol.xyz),
-                    O.Basis.build(M.basis_text(AUX), mol.symbols, mol.xyz))
+    return hf.DfTensor(b, a), O.df_build(O.Basis.build(M.basis_text(basis), mol.symbols, mol.xyz),
+                                         O.Basis.build(M.basis_text(AUX), mol.symbols, mol.xyz))
+
+
+@pytest.fixture(scope="module", params=sorted(MOLECULES))
+def system(hf, request):
+    df, bt = factors(hf, *MOLECULES[request.param])
+    yield df, bt
+    df.close()
+
+
+@pytest.fixture(scope="module", params=sorted(LARGE))
+def large_system(hf, request):
+    df, bt = factors(hf, *LARGE[request.param])
+    assert (df.n + 15) // 16 > 10
     yield df, bt
     df.close()
 
 
 @pytest.mark.parametrize("o", [1, 5, 16, 17, 48, 100, 160, 161, 330])
 def test_exchange_over_tiles(system, o):
-    df, bt = system
+    check_exchange(*system, o)
+
+
+@pytest.mark.parametrize("o", [17, 160, 161])
+def test_exchange_over_several_column_tiles(large_system, o):
+    check_exchange(*large_system, o)
+
+
+def check_exchange(df, bt, o):
     c = np.random.default_rng(100 + o).standard_normal((df.n, o)) / np.sqrt(df.n)
     j, k, _ = df.jk_precision(c, "fp64")
     jr, kr = O.df_jk(bt, df.n, c)
