@@ -121,8 +121,8 @@ def df_report(hf, M, steps=5, solves=True, basis="cc-pvdz"):
     def2-universal-JKFIT auxiliary basis (Cartesian), 160 occupied orbitals
     (random, fixed seed): the exchange contraction in FP64, FP32 and split
     BF16 on the matrix cores, each with its error against FP64.  At cc-pVTZ
-    the factor is kept packed ([rank][n(n+1)/2], 74 GB) and formed one
-    column chunk at a time."""
+    the factor (tiles of its rows' lower triangles, 75 GB) is formed one chunk
+    of tile rows at a time."""
     mol = M.water_cluster((4, 4, 2), seed=4)
     b = hf.Basis.from_g94(M.basis_text(basis), mol.symbols, mol.xyz)
     a = hf.Basis.from_g94(M.basis_text("def2-universal-jkfit"), mol.symbols, mol.xyz)
@@ -566,7 +566,7 @@ def main():
     ap.add_argument("--fock-steps", type=int, default=20)
     ap.add_argument("--solve-repeats", type=int, default=5)
     ap.add_argument("--no-df", action="store_true")
-    ap.add_argument("--no-df4", action="store_true", help="skip the config-4 DF (cc-pVTZ, packed factor)")
+    ap.add_argument("--no-df4", action="store_true", help="skip the config-4 DF (cc-pVTZ)")
     ap.add_argument("--only-df4", action="store_true",
                     help="only the config-4 DF build and DF J/K builds, without solves (profiling runs)")
     ap.add_argument("--no-cpu", action="store_true")

@@ -1,4 +1,6 @@
-// block_grid.h -- launch shape of the block kernels (engine.hip, grad.hip).
+// block_grid.h -- launch shape of the block kernels (engine.hip).  (The gradient's
+// own, grad.hip, stay at 64 threads: with 256, (fd|dd) asks for a larger private
+// segment.)
 #pragma once
 
 namespace hfg {

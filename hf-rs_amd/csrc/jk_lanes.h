@@ -1,12 +1,14 @@
 // jk_lanes.h -- the class launches of a J/K build over four streams.
 //
 // The 21 class kernels of a build are independent.  Where they do not fill the
-// chip (a small molecule, the last molecules of a served set) their latencies
-// would add up on one or two streams, and where they do, each kernel's last
+// chip (a small molecule) their latencies would add up on one or two streams, and where they do, each kernel's last
 // workgroups leave room for the next lane's: a process has four hardware queues,
 // so four lanes.  Each class goes to the lane with the least time so far, longest
 // class first, by an estimate of 50 us a kernel and 0.1 us a primitive step of
-// its longest job's waves and of its share of 2048 resident waves.
+// its longest job's waves and of its share of 2048 resident waves.  A batch's
+// builds run so, and the captured graph of one molecule's, which is made at the
+// second build with one set of outputs: the first (water / 6-31G* 0.93 ms) is
+// launched over two streams.  A server keeps to two as well (bscf.hip).
 // Measured in the captured graph of a build, two streams -> four lanes: water /
 // 6-31G* 0.84 -> 0.56 ms, (H2O)4 / cc-pVDZ 1.79 -> 1.34, (H2O)8 4.16 -> 3.78,
 // (H2O)16 16.3 -> 15.9, C10H22 / def2-SVP 3.19 -> 2.75.

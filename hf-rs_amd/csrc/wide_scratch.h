@@ -5,10 +5,12 @@
 // waves x 256 CUs = 8.5 GB, kept by that queue.  A process has four hardware queues
 // and about 32 GiB of address space for all their segments; the streams of several
 // contexts are dealt over all four, and once each holds what (dd|dd) asks for
-// (10,164 bytes, 5.3 GB), growing them one after another to 8.5 GB finds no room
-// in the end: the launch fails with HSA_STATUS_ERROR_OUT_OF_RESOURCES.  Kernels beyond (dd|dd)'s segment
-// therefore run on one stream of the device, kept until the process ends, between
-// events of the caller's: 3 x 5.3 + 8.5 GB.
+// (10,200 bytes, 5.3 GB), growing them one after another to 8.5 GB finds no room
+// in the end: the launch fails with HSA_STATUS_ERROR_OUT_OF_RESOURCES.  Kernels
+// beyond 10,240 bytes therefore run on one stream of the device, kept until the
+// process ends, between events of the caller's: 3 x 5.4 + 8.5 GB.  They are chosen
+// by class where they are launched; tests/test_private_segments.py checks the built
+// kernels against the limit.
 #pragma once
 #include <hip/hip_runtime.h>
 
