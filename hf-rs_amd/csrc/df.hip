@@ -525,21 +525,28 @@ struct DfEngine {
     }
   }
 
+  // The workspace of a jk() call (each buffer with a test of its own: an
+  // allocation before it may be the one that succeeded).
+  void reserve(int o, int precision) {
+    if (!d_q.p) d_q.alloc((size_t)rank * 8);
+    if (!d_tj.p) d_tj.alloc(2 * npt * 8);
+    if (precision != 0 && !d_P.p) d_P.alloc((size_t)n * n * 8);
+    df_exchange_reserve(rank, n, o, precision, precision == 0, xwork);
+  }
+
   // J = sum_Q B_Q (B_Q . P), P = 2 C C^T; K = 2 sum_Q (B_Q C)(B_Q C)^T
   // (src/df.rs:143-173), the exchange in the given precision (df_mfma.hip), J in
   // FP64.  dC: n x o device; outputs device n x n.  FP64 exchange gives
   // B_Q . P = 2 sum A_Q . C from its tiles; otherwise it is a pass over B.
   void jk(const double* dC, int o, double* dJ, double* dK, int precision) {
     const size_t nn = (size_t)n * n;
-    if (!d_q.p) d_q.alloc((size_t)rank * 8);
-    if (!d_tj.p) d_tj.alloc(2 * npt * 8);  // (its own test: the allocation before may be the one that succeeded)
+    reserve(o, precision);
     double* dq = d_q.as<double>();
     double* tiled_p = d_tj.as<double>();
     double* tiled_j = tiled_p + npt;
     if (precision == 0) {
       df_exchange(d_B.as<double>(), npt, rank, n, dC, o, 0, dK, dq, xwork, stream);
     } else {
-      if (!d_P.p) d_P.alloc(nn * 8);
       double* P = d_P.as<double>();
       bl->gemm(false, true, n, n, o, 2.0, dC, o, dC, o, 0.0, P, n);
       hipLaunchKernelGGL(k_tile_sym2, dim3((unsigned)((npt + 255) / 256)), dim3(256), 0, stream, P, n, npt, tiled_p);
@@ -787,6 +794,7 @@ static int df_host_jk(hfg_df* df, const double* cocc, int nocc, double* j, doubl
     if (e.d_io.bytes < (2 * nn + no) * 8) e.d_io.alloc((2 * nn + no) * 8);
     double *dj = e.d_io.as<double>(), *dk = dj + nn, *dc = dk + nn;
     upload(dc, cocc, no, e.stream);
+    e.reserve(nocc, precision);  // not between the events
     hipEvent_t ev[2] = {};
     struct Events {
       hipEvent_t* ev;

@@ -497,32 +497,41 @@ __global__ __launch_bounds__(256) void k_syrk_reduce(const P* __restrict__ part,
   if (i0 + c < j0 + r && j0 + r < n) K[(size_t)(j0 + r) * n + i0 + c] = tile[c][r];
 }
 
+// The launches' shapes, with the workspace for them.
+struct Shape {
+  int nt, nb = 0, gy = 0, tiles = 0;
+  long long L, steps, S;
+};
+template <class T>
+Shape k_reserve(int rank, int n, int o, bool gamma, ExchangeWork& w) {
+  Shape h;
+  h.nt = tiles_of(n);
+  column_tiles(o, h.nb, h.gy);
+  h.L = (long long)rank * o;
+  h.steps = (h.L + T::XK - 1) / T::XK;
+  if (h.steps > INT32_MAX) throw HfgError{HFG_UNSUPPORTED, "DF exchange: contraction index out of range"};
+  for (int r = 0; ROWS * r < n; ++r) h.tiles += syrk_tiles(n, r);
+  // slices: about six rounds of the chip's 512 workgroups (two a CU), at least
+  // four steps each, a multiple of 8
+  h.S = (3072 + h.tiles - 1) / h.tiles;
+  h.S = std::min(h.S, std::max<long long>(1, h.steps / 4));
+  h.S = (h.S + 7) / 8 * 8;
+  w.c.grow((size_t)h.gy * h.nt * 16 * h.nb * T::CH * 16);
+  w.x.grow((size_t)h.steps * n * 256);
+  w.part.grow((size_t)h.S * n * n * sizeof(typename T::P));
+  if (gamma) w.sums.grow((size_t)rank * h.nt * 2 * h.gy * 8);
+  return h;
+}
+
 template <class T>
 void k_from_tiles(const double* Bt, size_t npt, int rank, int n, const double* C, int o, double* K, double* gamma,
                   ExchangeWork& w, hipStream_t st) {
   typedef typename T::X X;
   typedef typename T::P P;
-  const int nt = tiles_of(n);
-  int nb = 0, gy = 0;
-  column_tiles(o, nb, gy);
-  const int an = 16 * nb;
-  const long long L = (long long)rank * o, steps = (L + T::XK - 1) / T::XK;
-  if (steps > INT32_MAX) throw HfgError{HFG_UNSUPPORTED, "DF exchange: contraction index out of range"};
-  int tiles = 0;
-  for (int r = 0; ROWS * r < n; ++r) tiles += syrk_tiles(n, r);
-  // slices: about six rounds of the chip's 512 workgroups (two a CU), at least
-  // four steps each, a multiple of 8
-  long long S = (3072 + tiles - 1) / tiles;
-  S = std::min(S, std::max<long long>(1, steps / 4));
-  S = (S + 7) / 8 * 8;
-  w.c.grow((size_t)gy * nt * an * T::CH * 16);
-  w.x.grow((size_t)steps * n * 256);
-  w.part.grow((size_t)S * n * n * sizeof(P));
-  double* part = nullptr;
-  if (gamma) {
-    w.sums.grow((size_t)rank * nt * 2 * gy * 8);
-    part = w.sums.template as<double>();
-  }
+  const Shape h = k_reserve<T>(rank, n, o, gamma != nullptr, w);
+  const int nt = h.nt, nb = h.nb, gy = h.gy, tiles = h.tiles, an = 16 * nb;
+  const long long L = h.L, steps = h.steps, S = h.S;
+  double* part = gamma ? w.sums.template as<double>() : nullptr;
   u4* cp = w.c.template as<u4>();
   X* x = w.x.template as<X>();
   hipLaunchKernelGGL(k_pack_c<T>, dim3((unsigned)((gy * nt * an * 16 + 255) / 256)), dim3(256), 0, st, C, n, o, nt, an,
@@ -547,6 +556,15 @@ void k_from_tiles(const double* Bt, size_t npt, int rank, int n, const double* C
 }
 
 }  // namespace
+
+void df_exchange_reserve(int rank, int n, int o, int precision, bool gamma, ExchangeWork& w) {
+  if (precision == 0)
+    k_reserve<F64>(rank, n, o, gamma, w);
+  else if (precision == 1)
+    k_reserve<F32>(rank, n, o, gamma, w);
+  else
+    k_reserve<BF16x3>(rank, n, o, gamma, w);
+}
 
 void df_exchange(const double* Bt, size_t npt, int rank, int n, const double* C, int o, int precision, double* K,
                  double* gamma, ExchangeWork& w, hipStream_t st) {

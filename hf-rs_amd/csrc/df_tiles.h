@@ -50,5 +50,7 @@ struct ExchangeWork {
 // gamma[Q] = 2 tr(B_Q C C^T).  On stream st.
 void df_exchange(const double* Bt, size_t npt, int rank, int n, const double* C, int o, int precision, double* K,
                  double* gamma, ExchangeWork& w, hipStream_t st);
+// Grows the workspace to what such a call needs, which then allocates nothing.
+void df_exchange_reserve(int rank, int n, int o, int precision, bool gamma, ExchangeWork& w);
 
 }  // namespace hfg

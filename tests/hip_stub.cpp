@@ -21,8 +21,9 @@ std::map<const void*, size_t> lds_limit;          // hipFuncSetAttribute
 std::string fail_kernel, watch_kernel;
 int watch_arg = 0;
 long fail_malloc = 0;                             // the k-th next hipMalloc fails (0: none)
-long counts[8];                                   // see stub_count
+long counts[9];                                   // see stub_count
 std::set<void*> watched_streams;
+bool recording = false;                           // an odd number of events recorded: BETWEEN counts allocations
 thread_local int last = 0;
 
 int failed(int code) { return last = code; }
@@ -46,10 +47,10 @@ thread_local struct {
 
 extern "C" {
 
-enum { MALLOCS, STREAMS, WATCHED, WATCHED_OUTSIDE, LDS_BEYOND, FAILED };
+enum { MALLOCS, STREAMS, WATCHED, WATCHED_OUTSIDE, LDS_BEYOND, FAILED, WATCHED_STREAMS, BETWEEN };
 long stub_count(int what) {
   std::lock_guard<std::mutex> lk(mu);
-  return what == 6 ? (long)watched_streams.size() : counts[what];
+  return what == WATCHED_STREAMS ? (long)watched_streams.size() : counts[what];
 }
 // The k-th next hipMalloc fails (0: none).
 void stub_fail_malloc(long k) {
@@ -74,6 +75,7 @@ void stub_watch(const char* name, int arg) {
 int hipMalloc(void** p, size_t bytes) {
   std::lock_guard<std::mutex> lk(mu);
   ++counts[MALLOCS];
+  if (recording) ++counts[BETWEEN];
   if (fail_malloc > 0 && --fail_malloc == 0) {
     ++counts[FAILED];
     *p = nullptr;
@@ -141,7 +143,11 @@ int hipEventDestroy(void* e) {
   free(e);
   return 0;
 }
-int hipEventRecord(void*, void*) { return 0; }
+int hipEventRecord(void*, void*) {
+  std::lock_guard<std::mutex> lk(mu);
+  recording = !recording;
+  return 0;
+}
 int hipEventSynchronize(void*) { return 0; }
 int hipEventElapsedTime(float* ms, void*, void*) {
   *ms = 1.f;

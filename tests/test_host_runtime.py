@@ -19,7 +19,7 @@ hf = entry._load()
 import molecules as M
 stub = C.CDLL({stub!r})
 stub.stub_count.restype = C.c_long
-MALLOCS, STREAMS, WATCHED, OUTSIDE, LDS_BEYOND, FAILED, WATCHED_STREAMS = range(7)
+MALLOCS, STREAMS, WATCHED, OUTSIDE, LDS_BEYOND, FAILED, WATCHED_STREAMS, BETWEEN = range(8)
 def basis(mol, name):
     return hf.Basis.from_g94(M.basis_text(name), mol.symbols, mol.xyz)
 def raises(code, call):
@@ -169,3 +169,17 @@ def test_lds_limit_of_a_kernel_is_shared_by_the_threads(program):
         a.contract_jk(np.eye(large.n))
     assert stub.stub_count(LDS_BEYOND) == 0, stub.stub_count(LDS_BEYOND)
     """)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32", "bf16x3"])
+def test_df_device_time_holds_no_allocation(program, precision):
+    """The device time that a J/K call returns is the contraction's, on a handle's first call as on later ones: no
+    allocation lies between its two events."""
+    program("""
+    b, aux = basis(water, "sto-3g"), basis(water, "def2-svp-rifit")
+    df = hf.DfTensor(b, aux)
+    before = stub.stub_count(MALLOCS), stub.stub_count(BETWEEN)
+    df.jk_precision(np.ones((b.n, 5)), %r)
+    assert stub.stub_count(MALLOCS) > before[0]
+    assert stub.stub_count(BETWEEN) == before[1], stub.stub_count(BETWEEN) - before[1]
+    """ % precision)
